@@ -537,6 +537,8 @@ __device__ inline void coincident_dir(const StepParams& P, int pidx_i, int pidx_
 
 // FP64 pair evaluation from p's side with the reference's operation order.
 // d = minimg(x_q - x_p) exactly as BoundingBox::distance; adds p's share to F and pr.
+// CT = false leaves the contact laws out (no type pair has one).
+template <bool CT>
 __device__ inline void pair64(const StepParams& P, const PairLaw& E, int pidx_p, int spec_p, double sp_, int pidx_q,
                               int spec_q, double sq_, double d[3], double r2, uint32_t ts, uint32_t st_pair, double F[3],
                               double* pr) {
@@ -558,7 +560,7 @@ __device__ inline void pair64(const StepParams& P, const PairLaw& E, int pidx_p,
     if (!(r2 > E.rcut2 * sq(sigCore - E.xi) && r2 <= rc2)) return;
     f0 = sc_f0(sigCore, r2, E.xi, E.e0, E.ew) -
          (P.force_shifted ? sc_f0(sigCore, rc2, E.xi, E.e0, E.ew) * sqrt(rc2 / r2) : 0.0);
-  } else if (E.law == CIL_LAW_HZ || E.law == CIL_LAW_EA) {
+  } else if (CT && (E.law == CIL_LAW_HZ || E.law == CIL_LAW_EA)) {
     double r = sqrt(r2);
     if (!(r <= (si + sj) / 2)) return;
     contact = true;
@@ -572,7 +574,9 @@ __device__ inline void pair64(const StepParams& P, const PairLaw& E, int pidx_p,
     double h = hh >= 0.0 ? hh : 0.0;
     if (E.law == CIL_LAW_HZ) {
       double Ri = si / 2, Rj = sj / 2;
-      f0 = -(pow(h, 1.5) / (E.hzk * (sqrt((1 / Ri) + (1 / Rj)))));
+      // h sqrt(h) for the reference's pow(h, 1.5): within one ulp of it, a tenth of the instructions
+      // and half the kernel's registers
+      f0 = -((h * sqrt(h)) / (E.hzk * (sqrt((1 / Ri) + (1 / Rj)))));
     } else {
       f0 = -(h * (p_is_i ? E.ea_p : E.ea_q));
     }
@@ -681,8 +685,41 @@ __device__ inline int bucket_of(const StepParams& P, int t, int x, int y, int z)
   return t * P.nbins + b;
 }
 
-// Up to two z-segments of the bins bz+olo .. bz+ohi (olo <= ohi, span <= ns in z), split at
-// the periodic seam; 0 segments when a non-periodic box clips the range away.
+// Up to two segments of the bins b+olo .. b+ohi of dimension d (olo <= ohi, span <= ns), split
+// at the periodic seam, in visiting order: segment k covers bins z0[k]..z1[k], whose unwrapped
+// offset from b starts at off[k].  0 segments when a non-periodic box clips the range away.
+__device__ inline int run_segments(const StepParams& P, int d, int b, int olo, int ohi, int* z0, int* z1, int* off) {
+  const int nz = P.ns[d];
+  int lo = b + olo, hi = b + ohi;
+  if (!P.box.pbc[d]) {
+    lo = lo < 0 ? 0 : lo;
+    hi = hi > nz - 1 ? nz - 1 : hi;
+    if (lo > hi) return 0;
+    z0[0] = lo; z1[0] = hi; off[0] = lo - b;
+    return 1;
+  }
+  if (hi < 0) {
+    z0[0] = lo + nz; z1[0] = hi + nz; off[0] = lo - b;
+    return 1;
+  }
+  if (lo > nz - 1) {
+    z0[0] = lo - nz; z1[0] = hi - nz; off[0] = lo - b;
+    return 1;
+  }
+  if (lo < 0) {
+    z0[0] = lo + nz; z1[0] = nz - 1; off[0] = lo - b;
+    z0[1] = 0; z1[1] = hi; off[1] = -b;
+    return 2;
+  }
+  if (hi > nz - 1) {
+    z0[0] = lo; z1[0] = nz - 1; off[0] = lo - b;
+    z0[1] = 0; z1[1] = hi - nz; off[1] = nz - b;
+    return 2;
+  }
+  z0[0] = lo; z1[0] = hi; off[0] = lo - b;
+  return 1;
+}
+// The same of a 3D stencil column's z range; a 2D column is one bin.
 __device__ inline int z_segments_range(const StepParams& P, int bz, int olo, int ohi, int* z0, int* z1, int* off) {
   if (P.box.dim != 3) {
     z0[0] = 0;
@@ -690,35 +727,7 @@ __device__ inline int z_segments_range(const StepParams& P, int bz, int olo, int
     off[0] = 0;
     return 1;
   }
-  const int nz = P.ns[2];
-  int lo = bz + olo, hi = bz + ohi;
-  if (!P.box.pbc[2]) {
-    lo = lo < 0 ? 0 : lo;
-    hi = hi > nz - 1 ? nz - 1 : hi;
-    if (lo > hi) return 0;
-    z0[0] = lo; z1[0] = hi; off[0] = lo - bz;
-    return 1;
-  }
-  if (hi < 0) {
-    z0[0] = lo + nz; z1[0] = hi + nz; off[0] = lo - bz;
-    return 1;
-  }
-  if (lo > nz - 1) {
-    z0[0] = lo - nz; z1[0] = hi - nz; off[0] = lo - bz;
-    return 1;
-  }
-  if (lo < 0) {
-    z0[0] = lo + nz; z1[0] = nz - 1; off[0] = lo - bz;
-    z0[1] = 0; z1[1] = hi; off[1] = -bz;
-    return 2;
-  }
-  if (hi > nz - 1) {
-    z0[0] = lo; z1[0] = nz - 1; off[0] = lo - bz;
-    z0[1] = 0; z1[1] = hi - nz; off[1] = nz - bz;
-    return 2;
-  }
-  z0[0] = lo; z1[0] = hi; off[0] = lo - bz;
-  return 1;
+  return run_segments(P, 2, bz, olo, ohi, z0, z1, off);
 }
 
 // Up to two z-segments of the stencil column [bz-R, bz+R] (split at the periodic seam).
@@ -754,7 +763,197 @@ __device__ inline int z_segments(const StepParams& P, int bz, int R, int* z0, in
   return 1;
 }
 
+// Wave w of the per-type layout: the sorted array is type-major; each element type's range is
+// cut into chunks of `per` particles, one per wave, so the type is wave-uniform.  False beyond
+// the last chunk.
+__device__ inline bool wave_type_chunk(const StepParams& P, const int* __restrict__ start, int w, int per, int* tp_out,
+                                       int* k0_out, int* k1_out) {
+  int tp = -1, k0 = 0, k1 = 0, acc = 0;
+  for (int t = 0; t < P.ntypes; ++t) {
+    const int T0 = start[t * P.nbins], T1 = start[(t + 1) * P.nbins];
+    const int nw = (T1 - T0 + per - 1) / per;
+    if (tp < 0 && w < acc + nw) {
+      tp = t;
+      k0 = T0 + (w - acc) * per;
+      k1 = T1;
+    }
+    acc += nw;
+  }
+  if (tp < 0) return false;
+  *tp_out = __builtin_amdgcn_readfirstlane(tp);
+  *k0_out = k0;
+  *k1_out = k1;
+  return true;
+}
+
+// Sum over the aligned group of `lanes` lanes (a power of two); every lane gets it.  The tree is
+// fixed, so the sum does not depend on timing.
 template <typename T>
+__device__ inline T group_sum(T v, int lanes) {
+  for (int o = lanes >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
+  return v;
+}
+
+// FP64 pair forces.  2^pair_shift lanes share one particle: they take its stencil columns in turn
+// (2D: the runs of bins along y at each x offset; 3D: along z at each (x, y) offset), and their
+// partial sums are added in a fixed tree.  Columns and runs are culled by the particle's own
+// cut-off; each candidate in turn gets a conservative distance test, and the survivors the
+// reference's predicate and arithmetic (pair64).  Four candidates are loaded together.
+// CT: some type pair has a contact law (their code and registers stay out otherwise).
+// Bound by the latency of its dependent loads (bin starts, then candidates) where the colony is
+// small, hence several lanes per particle and one run per column.  One thread per particle over
+// single bins, with the minimum image's FP64 division for every candidate, took 76 us (4,000 discs
+// in 2D) and 1,143 us (30,011 in 3D); this takes 10.6 and 82 us.  Caps of 5 or 6 waves per SIMD
+// spill and are slower (3D: 130 and 277 us a step against 112).
+constexpr int PAIR64_UNROLL = 4;
+template <int D, bool CT>
+__device__ inline void k_pair64_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
+  const StepParams& P = *Pp;
+  const int* __restrict__ start = S.start;
+  const double4* __restrict__ spos = (const double4*)S.spos;
+  const int* __restrict__ smeta = S.smeta;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int sh = P.pair_shift, lanes = 1 << sh;
+  const int w = __builtin_amdgcn_readfirstlane(bid * (blockDim.x / WAVE) + threadIdx.x / WAVE);
+  int tp, k0, k1;
+  if (!wave_type_chunk(P, start, w, WAVE >> sh, &tp, &k0, &k1)) return;
+  const int k = k0 + (lane >> sh), sub = lane & (lanes - 1);
+  if (k >= k1) return;
+  const uint32_t ts = (uint32_t)step_ts(S);
+  const int nE = P.nE, cshift = nE - 1;  // cell = particle >> cshift (nE is 1 or 2)
+  const int spec_p = tp / nE;
+  const int pidx = smeta[k] >> 3, cell_p = pidx >> cshift;
+  const double4 me = spos[k];
+  int bc[3];
+  unpack_bin(P, S.sbin[k], bc);
+  // place in the bin, for the culls only; a disc outside an open box counts as at the edge of
+  // the bin that holds it
+  const double xg[3] = {me.x, me.y, me.z};
+  float loc[3] = {0.f, 0.f, 0.f}, wid[3] = {0.f, 0.f, 0.f};
+  bool one[3] = {false, false, false};  // a periodic dimension of one bin: never culled
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    wid[d] = (float)P.w[d];
+    loc[d] = fminf(fmaxf((float)(xg[d] - bc[d] * P.w[d]), 0.0f), wid[d]);
+    one[d] = P.reach[d] == 0 && P.box.pbc[d];
+  }
+  const bool any_one = one[0] || one[1] || one[2];
+  double F[3] = {0.0, 0.0, 0.0}, pr = 0.0;
+  for (int tq = 0; tq < P.ntypes; ++tq) {
+    const int Rx = P.reach_tt[tp][tq][0];
+    if (Rx < 0) continue;
+    const int Rm = D == 3 ? P.reach_tt[tp][tq][1] : 0, Rr = P.reach_tt[tp][tq][D - 1];
+    const PairLaw E = load_law(P, tp, tq);
+    const int spec_q = tq / nE;
+    const double rca = P.rca_tt[tp][tq], rcb = P.rcb_tt[tp][tq];
+    const float rcp = fmaf((float)rca, (float)(me.w + P.sigma_bound[tq]), (float)rcb) * 1.001f + 1e-6f;
+    const float rcp2 = rcp * rcp;
+    const int side = 2 * Rm + 1, ncol = (2 * Rx + 1) * side;
+    for (int c = sub; c < ncol; c += lanes) {
+      const int cx = D == 3 ? c / side : c;
+      const int ox = cx - Rx, oy = D == 3 ? c - cx * side - Rm : 0;
+      const float gx = one[0] ? 0.0f : (ox > 0 ? (float)ox * wid[0] - loc[0] : (ox < 0 ? loc[0] - (float)(ox + 1) * wid[0] : 0.0f));
+      float rem = rcp2 - (gx > 0.0f ? gx * gx : 0.0f);
+      int nx = bc[0] + ox;
+      // image shift of the column: x_q - x_p - shift is the minimum image wherever the pair can
+      // interact (a periodic dimension has one bin or at least 2 reach + 1)
+      double shift[3] = {0.0, 0.0, 0.0};
+      if (nx < 0 || nx >= P.ns[0]) {
+        if (!P.box.pbc[0]) continue;
+        shift[0] = nx < 0 ? P.box.L[0] : -P.box.L[0];
+        nx += nx < 0 ? P.ns[0] : -P.ns[0];
+      }
+      int row = nx;
+      if (D == 3) {
+        const float gy = one[1] ? 0.0f : (oy > 0 ? (float)oy * wid[1] - loc[1] : (oy < 0 ? loc[1] - (float)(oy + 1) * wid[1] : 0.0f));
+        rem -= gy > 0.0f ? gy * gy : 0.0f;
+        int ny = bc[1] + oy;
+        if (ny < 0 || ny >= P.ns[1]) {
+          if (!P.box.pbc[1]) continue;
+          shift[1] = ny < 0 ? P.box.L[1] : -P.box.L[1];
+          ny += ny < 0 ? P.ns[1] : -P.ns[1];
+        }
+        row = nx * P.ns[1] + ny;
+      }
+      if (rem < 0.0f) continue;
+      int lo = -Rr, hi = Rr;
+      if (!one[D - 1]) {
+        const float sr = sqrtf(rem), wr = wid[D - 1];
+        const int a = (int)floorf((loc[D - 1] + sr) / wr), b = (int)ceilf((loc[D - 1] - sr) / wr) - 1;
+        hi = a < Rr ? a : Rr;
+        lo = b > -Rr ? b : -Rr;
+        if (lo > hi) continue;
+      }
+      int z0[2], z1[2], zo[2];
+      const int nseg = run_segments(P, D - 1, bc[D - 1], lo, hi, z0, z1, zo);
+      const int base = tq * P.nbins + row * P.ns[D - 1];
+      for (int sg = 0; sg < nseg; ++sg) {
+        const int zr = bc[D - 1] + zo[sg];  // unwrapped first bin of the segment
+        shift[D - 1] = zr < 0 ? P.box.L[D - 1] : (zr >= P.ns[D - 1] ? -P.box.L[D - 1] : 0.0);
+        const int j1 = start[base + z1[sg] + 1];
+        for (int j = start[base + z0[sg]]; j < j1; j += PAIR64_UNROLL) {
+          double4 r[PAIR64_UNROLL];
+          int m[PAIR64_UNROLL];
+#pragma unroll
+          for (int q = 0; q < PAIR64_UNROLL; ++q) {
+            const int jj = j + q < j1 ? j + q : j1 - 1;
+            r[q] = spos[jj];
+            m[q] = smeta[jj];
+          }
+          auto delta = [&](const double4& rq, double d[3]) -> double {
+            const double x[3] = {rq.x - me.x, rq.y - me.y, rq.z - me.z};
+            double r2 = 0.0;
+#pragma unroll
+            for (int dd = 0; dd < D; ++dd) {
+              d[dd] = x[dd] - shift[dd];
+              if (any_one && one[dd]) d[dd] -= (double)nint(d[dd] / P.box.L[dd]) * P.box.L[dd];
+              r2 += sq(d[dd]);
+            }
+            return r2;
+          };
+          unsigned hits = 0;
+#pragma unroll
+          for (int q = 0; q < PAIR64_UNROLL; ++q) {
+            double d[3];
+            const double r2 = delta(r[q], d);
+            const double rc = rca * (r[q].w + me.w) + rcb;
+            const bool hit = j + q < j1 && !(r2 > rc * rc * 1.000001) && ((m[q] >> 3) >> cshift) != cell_p;
+            hits |= hit ? 1u << q : 0u;
+          }
+          while (hits) {  // one copy of the law code
+            const int q = __ffs(hits) - 1;
+            hits &= hits - 1;
+            double4 rq = r[0];
+            int mq = m[0];
+#pragma unroll
+            for (int u = 1; u < PAIR64_UNROLL; ++u) {
+              if (q == u) {
+                rq = r[u];
+                mq = m[u];
+              }
+            }
+            double d[3] = {0.0, 0.0, 0.0};
+            const double r2 = delta(rq, d);
+            pair64<CT>(P, E, pidx, spec_p, me.w, mq >> 3, spec_q, rq.w, d, r2, ts, force_stream(S, ST_PAIR), F, &pr);
+          }
+        }
+      }
+    }
+  }
+  double* fp = (double*)S.fpair;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const double f = group_sum(F[d], lanes);
+    if (sub == 0) fp[(size_t)d * S.P + k] = f;
+  }
+  if (CT && P.pressure) pr = group_sum(pr, lanes);
+  if (sub == 0) ((double*)S.ppair)[k] = pr;
+}
+template <int D, bool CT>
+__global__ void __launch_bounds__(256) k_pair64(const StepParams* __restrict__ Pp, Dev S) {
+  k_pair64_body<D, CT>(Pp, S, xcd_block_chunked(blockIdx.x, gridDim.x));
+}
+
 __device__ inline void k_pair_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
   const StepParams& P = *Pp;
   const int D = P.box.dim;
@@ -769,22 +968,16 @@ __device__ inline void k_pair_body(const StepParams* __restrict__ Pp, const Dev&
   const int spec_p = species_of_cell(P, cell_p);
   int bc[3];
   unpack_bin(P, S.sbin[k], bc);
-  T xp[4];
-  if constexpr (sizeof(T) == 4) {
-    float4 r = ((const float4*)S.spos)[k];
-    xp[0] = r.x; xp[1] = r.y; xp[2] = r.z; xp[3] = r.w;
-  } else {
-    double4 r = ((const double4*)S.spos)[k];
-    xp[0] = r.x; xp[1] = r.y; xp[2] = r.z; xp[3] = r.w;
-  }
-  T F[3] = {0, 0, 0};
-  T pr = 0;
+  const float4 me = ((const float4*)S.spos)[k];
+  const float xp[4] = {me.x, me.y, me.z, me.w};
+  float F[3] = {0, 0, 0};
+  float pr = 0;
   for (int tq = 0; tq < P.ntypes; ++tq) {
     const int Rx = P.reach_tt[tp][tq][0];
     if (Rx < 0) continue;
     const int Ry = P.reach_tt[tp][tq][1], Rz = D == 3 ? P.reach_tt[tp][tq][2] : 0;
     const PairLaw E = load_law(P, tp, tq);
-    const T rca = (T)P.rca_tt[tp][tq], rcb = (T)P.rcb_tt[tp][tq], margin = (T)(sizeof(T) == 4 ? 1.0001 : 1.000001);
+    const float rca = (float)P.rca_tt[tp][tq], rcb = (float)P.rcb_tt[tp][tq];
     int z0[2], z1[2], zo[2];
     const int nseg = z_segments(P, bc[2], Rz, z0, z1, zo);
     for (int ox = -Rx; ox <= Rx; ++ox) {
@@ -801,68 +994,43 @@ __device__ inline void k_pair_body(const StepParams* __restrict__ Pp, const Dev&
           const int j0 = S.start[u0], j1 = S.start[u1 + 1];
           int u = u0, jend = S.start[u0 + 1];
           int oz = zo[sg];
-          // p's position relative to the source bin's frame (FP32: bin-local coordinates)
-          T qx = 0, qy = 0, qz = 0;
-          if constexpr (sizeof(T) == 4) {
-            qx = xp[0] - (T)(ox * P.w[0]);
-            qy = xp[1] - (T)(oy * P.w[1]);
-            qz = xp[2] - (T)(oz * P.w[2]);
-          }
+          // p's position relative to the source bin's frame (bin-local coordinates)
+          const float qx = xp[0] - (float)(ox * P.w[0]), qy = xp[1] - (float)(oy * P.w[1]);
+          float qz = xp[2] - (float)(oz * P.w[2]);
           for (int j = j0; j < j1; ++j) {
             while (j >= jend) {  // crossed into the next z-bin of the run
               ++u;
               ++oz;
               jend = S.start[u + 1];
-              if constexpr (sizeof(T) == 4) qz -= (T)P.w[2];
+              qz -= (float)P.w[2];
             }
             const int mq = S.smeta[j];
             const int qidx = mq >> 3;
-            if constexpr (sizeof(T) == 4) {
-              const float4 r = ((const float4*)S.spos)[j];
-              float d[3] = {r.x - qx, r.y - qy, D == 3 ? r.z - qz : 0.0f};
-              if (P.reach[0] == 0 && P.box.pbc[0]) d[0] -= (float)P.box.L[0] * rintf(d[0] * (float)P.box.invL[0]);
-              if (P.reach[1] == 0 && P.box.pbc[1]) d[1] -= (float)P.box.L[1] * rintf(d[1] * (float)P.box.invL[1]);
-              if (D == 3 && P.reach[2] == 0 && P.box.pbc[2])
-                d[2] -= (float)P.box.L[2] * rintf(d[2] * (float)P.box.invL[2]);
-              const float r2 = fmaf(d[0], d[0], fmaf(d[1], d[1], d[2] * d[2]));
-              const float rc = fmaf(rca, r.w + xp[3], rcb);
-              if (r2 > rc * rc * margin || (qidx >> cshift) == cell_p) continue;
-              float Fl[3] = {F[0], F[1], F[2]};
-              float prl = pr;
-              pair32(P, S, E, pidx, spec_p, xp[3], qidx, species_of_cell(P, qidx >> cshift), r.w, d, r2, ts, Fl, &prl);
-              F[0] = Fl[0]; F[1] = Fl[1]; F[2] = Fl[2];
-              pr = prl;
-            } else {
-              const double4 r = ((const double4*)S.spos)[j];
-              double xq[3] = {r.x, r.y, r.z};
-              double d[3] = {0, 0, 0};
-              double r2 = 0.0;
-              for (int dd = 0; dd < D; ++dd) {
-                double x = xq[dd] - (double)xp[dd];
-                if (P.box.pbc[dd]) x -= (double)nint(x / P.box.L[dd]) * P.box.L[dd];
-                d[dd] = x;
-                r2 += sq(x);
-              }
-              const double rc = rca * (r.w + (double)xp[3]) + rcb;
-              if (r2 > rc * rc * margin || (qidx >> cshift) == cell_p) continue;
-              double Fl[3] = {(double)F[0], (double)F[1], (double)F[2]};
-              double prl = pr;
-              pair64(P, E, pidx, spec_p, (double)xp[3], qidx, species_of_cell(P, qidx >> cshift), r.w, d, r2, ts,
-                     force_stream(S, ST_PAIR), Fl, &prl);
-              F[0] = Fl[0]; F[1] = Fl[1]; F[2] = Fl[2];
-              pr = prl;
-            }
+            const float4 r = ((const float4*)S.spos)[j];
+            float d[3] = {r.x - qx, r.y - qy, D == 3 ? r.z - qz : 0.0f};
+            if (P.reach[0] == 0 && P.box.pbc[0]) d[0] -= (float)P.box.L[0] * rintf(d[0] * (float)P.box.invL[0]);
+            if (P.reach[1] == 0 && P.box.pbc[1]) d[1] -= (float)P.box.L[1] * rintf(d[1] * (float)P.box.invL[1]);
+            if (D == 3 && P.reach[2] == 0 && P.box.pbc[2])
+              d[2] -= (float)P.box.L[2] * rintf(d[2] * (float)P.box.invL[2]);
+            const float r2 = fmaf(d[0], d[0], fmaf(d[1], d[1], d[2] * d[2]));
+            const float rc = fmaf(rca, r.w + xp[3], rcb);
+            if (r2 > rc * rc * 1.0001f || (qidx >> cshift) == cell_p) continue;
+            float Fl[3] = {F[0], F[1], F[2]};
+            float prl = pr;
+            pair32(P, S, E, pidx, spec_p, xp[3], qidx, species_of_cell(P, qidx >> cshift), r.w, d, r2, ts, Fl, &prl);
+            F[0] = Fl[0]; F[1] = Fl[1]; F[2] = Fl[2];
+            pr = prl;
           }
         }
       }
     }
   }
-  T* fp = (T*)S.fpair;
+  float* fp = (float*)S.fpair;
   for (int dd = 0; dd < D; ++dd) fp[(size_t)dd * S.P + k] = F[dd];
-  ((T*)S.ppair)[k] = pr;
+  ((float*)S.ppair)[k] = pr;
 }
-template <typename T>
-__global__ void __launch_bounds__(256) k_pair(const StepParams* __restrict__ Pp, Dev S) { k_pair_body<T>(Pp, S, xcd_block_chunked(blockIdx.x, gridDim.x)); }
+// Generic FP32 kernel (pair kernel variant 1).
+__global__ void __launch_bounds__(256) k_pair(const StepParams* __restrict__ Pp, Dev S) { k_pair_body(Pp, S, xcd_block_chunked(blockIdx.x, gridDim.x)); }
 
 // Lean FP32 pair kernel (fast mode), specialised on the dimension.  Waves are laid out per
 // element type (the sorted array is type-major), so the target type, its species, the law
@@ -1030,20 +1198,8 @@ __device__ inline void k_pair32_body(const StepParams* __restrict__ Pp, const De
   const int* __restrict__ start = S.start;
   const int lane = threadIdx.x & (WAVE - 1);
   const int w = __builtin_amdgcn_readfirstlane(bid * (blockDim.x / WAVE) + threadIdx.x / WAVE);
-  // wave -> (type, chunk of that type's sorted range)
-  int tp = -1, k0 = 0, k1 = 0, acc = 0;
-  for (int t = 0; t < P.ntypes; ++t) {
-    const int T0 = start[t * P.nbins], T1 = start[(t + 1) * P.nbins];
-    const int nw = (T1 - T0 + WAVE - 1) / WAVE;
-    if (tp < 0 && w < acc + nw) {
-      tp = t;
-      k0 = T0 + (w - acc) * WAVE;
-      k1 = T1;
-    }
-    acc += nw;
-  }
-  if (tp < 0) return;
-  tp = __builtin_amdgcn_readfirstlane(tp);
+  int tp, k0, k1;
+  if (!wave_type_chunk(P, start, w, WAVE, &tp, &k0, &k1)) return;
   const int k = k0 + lane;
   if (k >= k1) return;
   const uint32_t ts = (uint32_t)step_ts(S);

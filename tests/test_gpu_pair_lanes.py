@@ -1,0 +1,64 @@
+"""The stencil pair kernels with every number of lanes per particle, against the CPU oracle.
+
+The lanes per particle follow the context's particle slots, so a large capacity puts a small colony
+on the path of a large one.  Colonies: one particle, a partial last wave in each type, a box of one
+bin, a box at the smallest stencil grid, and an open box with discs outside it (kept in the edge
+bins until the drain takes them).  FP64 bar: 1e-12 of (sum of |pair terms| + |F|), as everywhere.
+"""
+import numpy as np
+import pytest
+
+from cil_cuda_amd import abi, configs
+from cil_cuda_amd.colony import Colony, HipMD
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _colony(dim, n, L, periodic, law, capacity, seed, stray=0):
+    rng = np.random.default_rng(seed)
+    p = configs.base_params(dim, 2, 1)
+    for s in range(2):
+        p.species[s].sig_well[0] = 0.5 + 0.2 * s
+        p.species[s].eps_core[0] = 10.0
+        p.species[s].eps_well[0] = 1.0
+    p.species[1].cross_adhesion = 0.5
+    configs.set_law(p, law, 2.0 if law == abi.LAW_LJ else 1.0)
+    p.pressure = 1
+    box = configs.make_box([L] * dim, [periodic] * dim)
+    counts = [n - n // 2, n // 2]
+    col = Colony(dim, 1, [capacity - capacity // 2, capacity // 2], ncells=counts)
+    for sp, m in zip(col.species, counts):
+        sp["pos"][:m, 0] = rng.uniform(0, L, (m, dim))
+        sp["sigma"][:m] = rng.uniform(0.8, 1.25, (m, 1))
+        sp["state"][:m] = abi.CS_CRAWLING
+        k = min(stray, m)  # outside an open box, some near each other
+        sp["pos"][:k, 0, dim - 1] = rng.uniform(-3.0, 0.2, k)
+        sp["pos"][:k, 0, 0] = rng.uniform(L - 0.5, L + 1.5, k)
+    return p, box, col
+
+
+CAPS = {2: (400, 50000, 100000, 200000), 3: (400, 10000, 20000, 40000, 80000)}
+
+
+@pytest.mark.parametrize("law", [abi.LAW_LJ, abi.LAW_SC, abi.LAW_HZ])
+@pytest.mark.parametrize("dim,cap", [(d, c) for d in (2, 3) for c in CAPS[d]])
+def test_pair_lanes_fp64(gpu, dim, cap, law):
+    cases = [(1, 12.0, 1, 0), (67, 9.0, 1, 0), (300, 2.2, 1, 0), (300, 5.0, 1, 0), (391, 9.0, 0, 40)]
+    for n, L, periodic, stray in cases:
+        p, box, col = _colony(dim, n, L, periodic, law, cap, seed=100 + n + law, stray=stray)
+        orc = O.Oracle(p, box, traversal=1)
+        ref = col.copy()
+        orc.forces(ref, 0)
+        scale = orc.force_scale(ref)
+        orc.close()
+        md = HipMD(p, box, [sp["capacity"] for sp in col.species])
+        md.upload(col)
+        frc, pr = md.forces()
+        md.close()
+        fref, prr = ref.flat("frc").reshape(-1, dim), ref.flat("pressure")
+        err = np.linalg.norm(frc - fref, axis=1)
+        worst = float(np.max(err / (1e-12 * (scale + np.linalg.norm(fref, axis=1)) + 1e-300)))
+        assert worst <= 1.0, (n, L, periodic, worst)
+        if law == abi.LAW_HZ:
+            assert np.allclose(pr, prr, rtol=1e-11, atol=1e-11 * max(1.0, float(np.max(np.abs(prr)))))
