@@ -1032,12 +1032,11 @@ __device__ inline void k_pair_body(const StepParams* __restrict__ Pp, const Dev&
 // Generic FP32 kernel (pair kernel variant 1).
 __global__ void __launch_bounds__(256) k_pair(const StepParams* __restrict__ Pp, Dev S) { k_pair_body(Pp, S, xcd_block_chunked(blockIdx.x, gridDim.x)); }
 
-// Lean FP32 pair kernel (fast mode), specialised on the dimension.  Waves are laid out per
-// element type (the sorted array is type-major), so the target type, its species, the law
-// of each (target, source) type pair, the stencil reach and the cross-adhesion choice are
-// wave-uniform (scalar registers).  Same traversal and pair semantics as k_pair<float>.
-// Single-disc cells: the same-cell exclusion is j == k, so the inner loop reads only the
-// 16-byte sorted record of each candidate.
+// Lean FP32 pair kernel (k_pair32, fast mode), specialised on the dimension.  Waves are laid out
+// per element type (the sorted array is type-major), so the target type, its species, the law of
+// each (target, source) type pair, the stencil reach and the cross-adhesion choice are wave-uniform
+// (scalar registers).  Single-disc cells: the same-cell exclusion is j == k, so the inner loop
+// reads only each candidate's sorted record and packed bin.
 // Law coefficients of one (target, source) element-type pair for the FP32 kernels.
 struct Law32 {
   int law;
@@ -1077,10 +1076,11 @@ constexpr int LC_ANY = -1, LC_CONTACT = 100;
 // One pair term of the FP32 kernels (LJParams / SCParams::elemForce, MD.cuh:89-110,190-207;
 // contact laws with the device semantics of MD.cu:317-362, canonical i = lower index).
 // Returns false when the pair adds nothing: outside the law's range, or an LJ pair inside the
-// 1e-5 cut-off guard band, which is recorded in gslot for the exact FP64 decision.  For a
+// 1e-5 cut-off guard band, which is recorded in gslot (the caller's GUARD_SLOTS entries) for the
+// exact FP64 decision.  For a
 // coincident 2D contact (dx, dy) become the reference's random direction.
 template <int D, int LC = LC_ANY>
-__device__ __forceinline__ bool pair_term32(const StepParams& P, const Dev& S, const Law32& L, int k, int j, int pidx,
+__device__ __forceinline__ bool pair_term32(const StepParams& P, const Dev& S, const Law32& L, int* gslot, int j, int pidx,
                                             float sp_, float sq_, float r2, uint32_t ts, float& dx, float& dy,
                                             int& nguard, float& f0, bool& contact, float& temp) {
   const float ssum = sq_ + sp_;
@@ -1093,7 +1093,7 @@ __device__ __forceinline__ bool pair_term32(const StepParams& P, const Dev& S, c
     const float rc2 = sij2 * L.rcut2;
     if (r2 > rc2 * 1.00001f) return false;
     if (r2 > rc2 * 0.99999f) {  // decided exactly in FP64 by guard_force after the pair loop
-      if (nguard < GUARD_SLOTS) S.gslot[(size_t)k * GUARD_SLOTS + nguard] = j;
+      if (nguard < GUARD_SLOTS) gslot[nguard] = j;
       ++nguard;
       return false;
     }
@@ -1154,15 +1154,15 @@ __device__ __forceinline__ bool pair_term32(const StepParams& P, const Dev& S, c
 
 // FP32 LJ pairs of sorted particle k that fell inside the 1e-5 cut-off guard band: the
 // exact FP64 cut-off decision (the reference's predicate) for each, and the FP32 force of
-// those inside, summed in gslot order into F.  Called by the FP32 pair kernels for their own
-// particle after its pair loop (positions are stable during the pass), so no separate pass
-// is launched; F's sum is then added to the pair sum, as one FP32 addition per component.
-__device__ inline void guard_force(const StepParams& P, const Dev& S, int k, int n, float F[3]) {
+// those inside, summed in gslot order (n recorded pairs) into F.  Called by the FP32 pair kernels
+// for their own particle after its pair loop (positions are stable during the pass), so no separate
+// pass is launched; F's sum is then added to the pair sum, as one FP32 addition per component.
+__device__ inline void guard_force(const StepParams& P, const Dev& S, int k, const int* gslot, int n, float F[3]) {
   const int D = P.box.dim;
   const int meta = S.smeta[k];
   const int pidx = meta >> 3, tp = meta & 7;
   for (int g = 0; g < n && g < GUARD_SLOTS; ++g) {
-    const int j = S.gslot[(size_t)k * GUARD_SLOTS + g];
+    const int j = gslot[g];
     const int mq = S.smeta[j];
     const int qidx = mq >> 3, tq = mq & 7;
     const LawEntry& A = P.law[tp][tq];
@@ -1190,17 +1190,29 @@ __device__ inline void guard_force(const StepParams& P, const Dev& S, int k, int
   }
 }
 
+// Bin coordinate along the run dimension (the fastest one) of a sorted slot's packed bin.
+template <int D>
+__device__ __forceinline__ int run_coord(int sb) { return D == 3 ? (sb & 1023) : (sb & 0xffff); }
+
+// Lanes, columns and runs as in k_pair64; a candidate's frame is its own bin's (FP32 local
+// coordinates), read from its packed bin beside its position, so a run crosses bins without a
+// look-up.  Lanes keep their own guard-band pairs (LDS) and resolve them before the sum.
+// At 131,071 particles (3D): 307 us with one thread per particle over single bins, 120 us with four.
+constexpr int PAIR32_UNROLL = 2;  // 4 need 98-112 VGPRs: 184 against 173 us per step
 template <int D>
 __device__ inline void k_pair32_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
+  __shared__ int guard[256][GUARD_SLOTS];  // each lane's pairs inside the LJ guard band
   const StepParams& P = *Pp;
   const float4* __restrict__ spos = (const float4*)S.spos;
   const int* __restrict__ smeta = S.smeta;
+  const int* __restrict__ sbin = S.sbin;
   const int* __restrict__ start = S.start;
   const int lane = threadIdx.x & (WAVE - 1);
+  const int sh = P.pair_shift, lanes = 1 << sh;
   const int w = __builtin_amdgcn_readfirstlane(bid * (blockDim.x / WAVE) + threadIdx.x / WAVE);
   int tp, k0, k1;
-  if (!wave_type_chunk(P, start, w, WAVE, &tp, &k0, &k1)) return;
-  const int k = k0 + lane;
+  if (!wave_type_chunk(P, start, w, WAVE >> sh, &tp, &k0, &k1)) return;
+  const int k = k0 + (lane >> sh), sub = lane & (lanes - 1);
   if (k >= k1) return;
   const uint32_t ts = (uint32_t)step_ts(S);
   const int nE = P.nE;
@@ -1210,83 +1222,102 @@ __device__ inline void k_pair32_body(const StepParams* __restrict__ Pp, const De
   const int pidx = smeta[k] >> 3;
   const int cell_p = pidx >> cshift;
   int bc[3];
-  unpack_bin(P, S.sbin[k], bc);
+  unpack_bin(P, sbin[k], bc);
   const float4 me = spos[k];
-  const float wx = (float)P.w[0], wy = (float)P.w[1], wz = (float)P.w[2];
-  const bool mix = P.reach[0] == 0 && P.box.pbc[0], miy = P.reach[1] == 0 && P.box.pbc[1];
-  const bool miz = D == 3 && P.reach[2] == 0 && P.box.pbc[2];
-  float Fx = 0.f, Fy = 0.f, Fz = 0.f, pr = 0.f;
+  // bin widths, and the place in the bin for the culls (a disc outside an open box counts as at
+  // the edge of the bin that holds it)
+  const float xl[3] = {me.x, me.y, me.z};
+  float loc[3] = {0.f, 0.f, 0.f}, wid[3] = {0.f, 0.f, 0.f};
+  bool one[3] = {false, false, false};  // a periodic dimension of one bin: minimum image per pair
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    wid[d] = (float)P.w[d];
+    loc[d] = fminf(fmaxf(xl[d], 0.0f), wid[d]);
+    one[d] = P.reach[d] == 0 && P.box.pbc[d];
+  }
+  const bool any_one = one[0] || one[1] || one[2];
+  const float wr = wid[D - 1], mr = xl[D - 1];
+  float F[3] = {0.f, 0.f, 0.f}, pr = 0.f;
   int nguard = 0;
   for (int tq = 0; tq < P.ntypes; ++tq) {
     const int Rx = P.reach_tt[tp][tq][0];
     if (Rx < 0) continue;
-    const int Ry = P.reach_tt[tp][tq][1], Rz = D == 3 ? P.reach_tt[tp][tq][2] : 0;
+    const int Rm = D == 3 ? P.reach_tt[tp][tq][1] : 0, Rr = P.reach_tt[tp][tq][D - 1];
     const Law32 Lw = law32(P, tp, tq);
     const float rca = (float)P.rca_tt[tp][tq], rcb = (float)P.rcb_tt[tp][tq];
     const float cadh = (tq / nE == spec_p) ? 1.0f : ca_p;  // scale for f0 >= 0 (MD.cu:345-360)
     const bool same_species_cells = nE == 2 && (tq / nE == spec_p);
-    const bool self_bucket = tq == tp;
     // This particle's largest cut-off against type tq (diameter bound of tq), with a margin
     // far above FP32 rounding: bins beyond it cannot hold a partner.  Columns are culled by
-    // their x/y gap and each z-run is clipped to the bins its remaining radius reaches.
+    // their x/y gap and each run is clipped to the bins its remaining radius reaches.
     const float rcp = fmaf(rca, me.w + (float)P.sigma_bound[tq], rcb) * 1.001f + 1e-6f;
     const float rcp2 = rcp * rcp;
-    int z0[2], z1[2], zo[2];
-    for (int ox = -Rx; ox <= Rx; ++ox) {
+    const int side = 2 * Rm + 1, ncol = (2 * Rx + 1) * side;
+    for (int c = sub; c < ncol; c += lanes) {
+      const int cx = D == 3 ? c / side : c;
+      const int ox = cx - Rx, oy = D == 3 ? c - cx * side - Rm : 0;
       int nx = bc[0] + ox;
       if (P.box.pbc[0]) nx = nx < 0 ? nx + P.ns[0] : (nx >= P.ns[0] ? nx - P.ns[0] : nx);
       else if (nx < 0 || nx >= P.ns[0]) continue;
-      const float qx = me.x - (float)ox * wx;
-      const float gx = mix ? 0.0f : (ox > 0 ? (float)ox * wx - me.x : (ox < 0 ? me.x - (float)(ox + 1) * wx : 0.0f));
-      const float gx2 = gx > 0.0f ? gx * gx : 0.0f;
-      if (gx2 > rcp2) continue;
-      for (int oy = -Ry; oy <= Ry; ++oy) {
+      const float qx = me.x - (float)ox * wid[0];
+      const float gx = one[0] ? 0.0f : (ox > 0 ? (float)ox * wid[0] - loc[0] : (ox < 0 ? loc[0] - (float)(ox + 1) * wid[0] : 0.0f));
+      float rem = rcp2 - (gx > 0.0f ? gx * gx : 0.0f), qy = 0.0f;
+      int row = nx;
+      if (D == 3) {
         int ny = bc[1] + oy;
         if (P.box.pbc[1]) ny = ny < 0 ? ny + P.ns[1] : (ny >= P.ns[1] ? ny - P.ns[1] : ny);
         else if (ny < 0 || ny >= P.ns[1]) continue;
-        const float qy = me.y - (float)oy * wy;
-        const float gy = miy ? 0.0f : (oy > 0 ? (float)oy * wy - me.y : (oy < 0 ? me.y - (float)(oy + 1) * wy : 0.0f));
-        const float rem = rcp2 - gx2 - (gy > 0.0f ? gy * gy : 0.0f);
-        if (rem < 0.0f) continue;
-        int zlo = -Rz, zhi = Rz;
-        if (D == 3 && !miz) {
-          const float sr = sqrtf(rem);
-          const int a = (int)floorf((me.z + sr) / wz), b = (int)ceilf((me.z - sr) / wz) - 1;
-          zhi = a < Rz ? a : Rz;
-          zlo = b > -Rz ? b : -Rz;
-          if (zlo > zhi) continue;
-        }
-        const int nseg = z_segments_range(P, bc[2], zlo, zhi, z0, z1, zo);
-        for (int sg = 0; sg < nseg; ++sg) {
-          const int u0 = bucket_of(P, tq, nx, ny, z0[sg]);
-          const int u1 = bucket_of(P, tq, nx, ny, z1[sg]);
-          const int j1 = start[u1 + 1];
-          int u = u0, jend = start[u0 + 1];
-          float qz = me.z - (float)zo[sg] * wz;
-          for (int j = start[u0]; j < j1; ++j) {
-            while (j >= jend) {
-              ++u;
-              jend = start[u + 1];
-              qz -= wz;
+        qy = me.y - (float)oy * wid[1];
+        const float gy = one[1] ? 0.0f : (oy > 0 ? (float)oy * wid[1] - loc[1] : (oy < 0 ? loc[1] - (float)(oy + 1) * wid[1] : 0.0f));
+        rem -= gy > 0.0f ? gy * gy : 0.0f;
+        row = nx * P.ns[1] + ny;
+      }
+      if (rem < 0.0f) continue;
+      int lo = -Rr, hi = Rr;
+      if (!one[D - 1]) {
+        const float sr = sqrtf(rem);
+        const int a = (int)floorf((loc[D - 1] + sr) / wr), b = (int)ceilf((loc[D - 1] - sr) / wr) - 1;
+        hi = a < Rr ? a : Rr;
+        lo = b > -Rr ? b : -Rr;
+        if (lo > hi) continue;
+      }
+      int z0[2], z1[2], zo[2];
+      const int nseg = run_segments(P, D - 1, bc[D - 1], lo, hi, z0, z1, zo);
+      const int base = tq * P.nbins + row * P.ns[D - 1];
+      for (int sg = 0; sg < nseg; ++sg) {
+        const int unwrap = zo[sg] - z0[sg];  // bin coordinate along the run -> offset from p's bin
+        const int j1 = start[base + z1[sg] + 1];
+        for (int j = start[base + z0[sg]]; j < j1; j += PAIR32_UNROLL) {
+          float4 r[PAIR32_UNROLL];
+          int sb[PAIR32_UNROLL];
+#pragma unroll
+          for (int q = 0; q < PAIR32_UNROLL; ++q) {
+            const int jj = j + q < j1 ? j + q : j1 - 1;
+            r[q] = spos[jj];
+            sb[q] = sbin[jj];
+          }
+#pragma unroll
+          for (int q = 0; q < PAIR32_UNROLL; ++q) {
+            const float qr = mr - (float)(run_coord<D>(sb[q]) + unwrap) * wr;
+            float dx = r[q].x - qx, dy = D == 3 ? r[q].y - qy : r[q].y - qr, dz = D == 3 ? r[q].z - qr : 0.0f;
+            if (any_one) {
+              if (one[0]) dx -= (float)P.box.L[0] * rintf(dx * (float)P.box.invL[0]);
+              if (one[1]) dy -= (float)P.box.L[1] * rintf(dy * (float)P.box.invL[1]);
+              if (D == 3 && one[2]) dz -= (float)P.box.L[2] * rintf(dz * (float)P.box.invL[2]);
             }
-            const float4 r = spos[j];
-            float dx = r.x - qx, dy = r.y - qy, dz = D == 3 ? r.z - qz : 0.0f;
-            if (mix) dx -= (float)P.box.L[0] * rintf(dx * (float)P.box.invL[0]);
-            if (miy) dy -= (float)P.box.L[1] * rintf(dy * (float)P.box.invL[1]);
-            if (miz) dz -= (float)P.box.L[2] * rintf(dz * (float)P.box.invL[2]);
             const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-            const float ssum = r.w + me.w;
+            const float ssum = r[q].w + me.w;
             const float rc = fmaf(rca, ssum, rcb);
-            if (r2 > rc * rc * 1.0001f) continue;
-            if (self_bucket && j == k) continue;
-            if (same_species_cells && ((smeta[j] >> 3) >> cshift) == cell_p) continue;
+            const int jq = j + q;
+            if (jq >= j1 || r2 > rc * rc * 1.0001f || jq == k) continue;
+            if (same_species_cells && ((smeta[jq] >> 3) >> cshift) == cell_p) continue;
             float f0, temp;
             bool contact;
-            if (!pair_term32<D>(P, S, Lw, k, j, pidx, me.w, r.w, r2, ts, dx, dy, nguard, f0, contact, temp)) continue;
+            if (!pair_term32<D>(P, S, Lw, guard[threadIdx.x], jq, pidx, me.w, r[q].w, r2, ts, dx, dy, nguard, f0, contact, temp)) continue;
             const float fs = f0 < 0.0f ? f0 : cadh * f0;
-            Fx = fmaf(fs, dx, Fx);
-            Fy = fmaf(fs, dy, Fy);
-            if (D == 3) Fz = fmaf(fs, dz, Fz);
+            F[0] = fmaf(fs, dx, F[0]);
+            F[1] = fmaf(fs, dy, F[1]);
+            if (D == 3) F[2] = fmaf(fs, dz, F[2]);
             if (contact && temp != 0.0f) pr -= fs / temp;
           }
         }
@@ -1295,25 +1326,24 @@ __device__ inline void k_pair32_body(const StepParams* __restrict__ Pp, const De
   }
   if (nguard > 0) {
     float g[3] = {0.f, 0.f, 0.f};
-    guard_force(P, S, k, nguard, g);
-    Fx += g[0];
-    Fy += g[1];
-    if (D == 3) Fz += g[2];
+    guard_force(P, S, k, guard[threadIdx.x], nguard, g);
+    for (int d = 0; d < D; ++d) F[d] += g[d];
   }
   float* fp = (float*)S.fpair;
-  fp[k] = Fx;
-  fp[(size_t)S.P + k] = Fy;
-  if (D == 3) fp[2 * (size_t)S.P + k] = Fz;
-  ((float*)S.ppair)[k] = P.pressure ? pr : 0.0f;
-  if (nguard > GUARD_SLOTS) atomicOr(S.err, (unsigned)ERR_GUARD);
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const float f = group_sum(F[d], lanes);
+    if (sub == 0) fp[(size_t)d * S.P + k] = f;
+  }
+  pr = P.pressure ? group_sum(pr, lanes) : 0.0f;
+  if (sub == 0) ((float*)S.ppair)[k] = pr;
+  if (group_sum(nguard, lanes) > GUARD_SLOTS) atomicOr(S.err, (unsigned)ERR_GUARD);
 }
+#define PAIR32_WPE 5  // six waves per SIMD spill
 template <int D>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PAIR32_WPE)))
 k_pair32(const StepParams* __restrict__ Pp, Dev S) { k_pair32_body<D>(Pp, S, xcd_block_chunked(blockIdx.x, gridDim.x)); }
 
-// LJ pairs whose FP32 distance fell within 1e-5 of the cut-off: exact FP64 decision
-// (LJParams::elemForce predicate r^2 <= RCUT^2 sigma_ij^2 on the canonical positions), then
-// the FP32 force added by the thread that owns the target particle (deterministic).
 // ======================================================================================
 // Neighbour-list mode (FP32).  A list entry is (sorted index << 10) | bin offset code; the
 // bins are sized for cut-off + skin, so the stencil reach is at most 4 and the offsets
@@ -1658,7 +1688,7 @@ __device__ __forceinline__ void list_segment(const StepParams& P, const Dev& S, 
     } else {
       float temp;
       bool contact;
-      if (!pair_term32<D, LC>(P, S, Lw, k, (int)(e >> 10), pidx, me.w, r.w, r2, ts, dx, dy, nguard, f0, contact,
+      if (!pair_term32<D, LC>(P, S, Lw, nullptr, (int)(e >> 10), pidx, me.w, r.w, r2, ts, dx, dy, nguard, f0, contact,
                               temp))
         return;
       const float fs = f0 < 0.0f ? f0 : cadh * f0;
@@ -1793,7 +1823,7 @@ __device__ inline void k_pair_list_body(const StepParams* __restrict__ Pp, const
   else run_types(std::false_type{});
   if (nguard > 0) {
     float g[3] = {0.f, 0.f, 0.f};
-    guard_force(P, S, k, nguard, g);
+    guard_force(P, S, k, S.gslot + (size_t)k * GUARD_SLOTS, nguard, g);
     Fx += g[0];
     Fy += g[1];
     if (D == 3) Fz += g[2];
