@@ -95,7 +95,7 @@ __device__ inline void k_keys_body(const StepParams* __restrict__ Pp, const Dev&
   }
   int b = bucket_key(P, p, s, x);
   S.key[p] = b;
-  S.rank[p] = atomicAdd(&S.count[b], 1);
+  atomicAdd(&S.count[b], 1);
 }
 __global__ void k_keys(const StepParams* __restrict__ Pp, Dev S) { k_keys_body(Pp, S, (int)blockIdx.x); }
 
@@ -171,8 +171,9 @@ __device__ inline int block_sum(int v, int* lds) {
 // Second pass: each 256-item block lies inside one scan tile t and adds the sum of the tile
 // totals before t (at most a few hundred, summed by the block itself); the block holding the
 // last item writes the grand total.  With n == 0 block 0 writes the total (0).
+// `cur` (may be null) gets a copy of the scan: the scatter's cursors.
 __device__ inline void k_scan_add_body(int* __restrict__ out, const int* __restrict__ bsum, int n,
-                                       int* __restrict__ total_out, int bid) {
+                                       int* __restrict__ total_out, int* __restrict__ cur, int bid) {
   __shared__ int lds[WAVE];
   const int i0 = bid * (int)blockDim.x;
   const int t = i0 / SCAN_TILE;
@@ -180,13 +181,17 @@ __device__ inline void k_scan_add_body(int* __restrict__ out, const int* __restr
   for (int q = (int)threadIdx.x; q < t; q += (int)blockDim.x) acc += bsum[q];
   acc = block_sum(acc, lds);
   const int i = i0 + (int)threadIdx.x;
-  if (i < n) out[i] += acc;
+  if (i < n) {
+    const int v = out[i] + acc;
+    out[i] = v;
+    if (cur) cur[i] = v;
+  }
   if (total_out && (n > 0 ? i == n - 1 : (bid == 0 && threadIdx.x == 0))) *total_out = acc + bsum[t];
 }
 __global__ void __launch_bounds__(256) k_scan_add(int* __restrict__ out, const int* __restrict__ bsum, int n,
-                                                  int* __restrict__ total_out, SortGate gate) {
+                                                  int* __restrict__ total_out, int* __restrict__ cur, SortGate gate) {
   if (gate_closed(gate)) return;
-  k_scan_add_body(out, bsum, n, total_out, (int)blockIdx.x);
+  k_scan_add_body(out, bsum, n, total_out, cur, (int)blockIdx.x);
 }
 
 // ======================================================================================
@@ -198,7 +203,7 @@ __device__ inline void k_scatter_body(const Dev& S, int bid) {
   if (p >= S.P) return;
   int b = S.key[p];
   if (b < 0) return;
-  S.idx[S.start[b] + S.rank[p]] = p;
+  S.idx[atomicAdd(&S.count[b], 1)] = p;  // the scan left the bucket's start in its count
 }
 __global__ void k_scatter(Dev S) { k_scatter_body(S, (int)blockIdx.x); }
 
@@ -400,6 +405,136 @@ __global__ void __launch_bounds__(WAVE* BINSORT_WAVES) k_binsort(const StepParam
 }
 
 // ======================================================================================
+// Bin sort of a small colony in one launch, without communication between its workgroups.
+// Workgroup b owns an equal share of the buckets: it sums the counts of all buckets before them,
+// scans its own, picks its particles out of all keys, and orders and writes them.  A kernel of a
+// captured step takes about 4.6 us however little it does, and the general sort's four took 19 us
+// at 4,000 particles in 27,000 buckets.  (One workgroup for everything takes 24 us there: a CU
+// handles about one scattered access per cycle, and a particle needs ten.)
+// The bucket counts are left as they are, since other workgroups may still read them: the pair
+// kernel that follows clears them (clear_counts).
+// ======================================================================================
+constexpr int SORTM_THREADS = 512;
+constexpr int SORTM_RANGE = 4 * SORTM_THREADS;  // buckets per workgroup, at most
+
+// Inclusive sum over the wave's lanes (data-parallel-primitive moves, no LDS traffic).
+__device__ __forceinline__ int wave_inclusive_sum(int x) {
+#define CIL_DPP_ADD(ctrl, rows) x += __builtin_amdgcn_update_dpp(0, x, ctrl, rows, 0xf, true)
+  CIL_DPP_ADD(0x111, 0xf);  // row_shr:1
+  CIL_DPP_ADD(0x112, 0xf);  // row_shr:2
+  CIL_DPP_ADD(0x114, 0xf);  // row_shr:4
+  CIL_DPP_ADD(0x118, 0xf);  // row_shr:8
+  CIL_DPP_ADD(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
+  CIL_DPP_ADD(0x143, 0xc);  // row_bcast:31 into rows 2 and 3
+#undef CIL_DPP_ADD
+  return x;
+}
+
+template <typename T>
+__device__ inline void k_sort_multi_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
+  const StepParams& P = *Pp;
+  constexpr int NW = SORTM_THREADS / WAVE;
+  __shared__ int st[SORTM_RANGE + 1], cur[SORTM_RANGE], wsum[NW], wpre[NW];
+  const int tid = (int)threadIdx.x, lane = tid & (WAVE - 1), wid = tid / WAVE;
+  const int n = P.nbuckets, range = P.sort_range;
+  const int lo = bid * range, hi = min(lo + range, n);  // range is a multiple of 4
+  // particles before this range
+  int sum = 0;
+  for (int u0 = 0; u0 < lo; u0 += 4 * 4 * SORTM_THREADS) {
+    int4 c[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int u = u0 + (q * SORTM_THREADS + tid) * 4;
+      c[q] = u < lo ? *reinterpret_cast<const int4*>(S.count + u) : make_int4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sum += c[q].x + c[q].y + c[q].z + c[q].w;
+  }
+  int v[4];
+  const int u = lo + tid * 4;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) v[q] = u + q < hi ? S.count[u + q] : 0;
+  const int own = v[0] + v[1] + v[2] + v[3];
+  const int inc = wave_inclusive_sum(own), pre = wave_inclusive_sum(sum);
+  if (lane == WAVE - 1) {
+    wsum[wid] = inc;
+    wpre[wid] = pre;
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) cur[tid * 4 + q] = 0;
+  __syncthreads();
+  int at = inc - own, end = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    at += wpre[w] + (w < wid ? wsum[w] : 0);
+    end += wpre[w] + wsum[w];
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    st[tid * 4 + q] = at;  // from hi on: the end of the range
+    if (u + q < hi) S.start[u + q] = at;
+    at += v[q];
+  }
+  if (tid == SORTM_THREADS - 1) {
+    st[SORTM_RANGE] = end;
+    if (hi == n) S.start[n] = end;
+  }
+  __syncthreads();
+  // this range's particles, in arrival order inside a bucket
+  for (int p0 = 0; p0 < S.P; p0 += 4 * SORTM_THREADS) {
+    int b[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int p = p0 + q * SORTM_THREADS + tid;
+      b[q] = p < S.P ? S.key[p] : -1;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (b[q] < lo || b[q] >= hi) continue;
+      const int l = b[q] - lo;
+      S.slot[st[l] + atomicAdd(&cur[l], 1)] = p0 + q * SORTM_THREADS + tid;
+    }
+  }
+  __syncthreads();
+  // each at its place by ascending particle index, as in the general sort
+  for (int k = st[0] + tid; k < end; k += SORTM_THREADS) {
+    const int p = S.slot[k], b = S.key[p], l = b - lo;
+    const int s0 = st[l], s1 = st[l + 1];
+    if (s1 - s0 > BINSORT_MAX) {
+      if (k == s0) atomicOr(S.err, (unsigned)ERR_BIN_OVERFLOW);
+      continue;
+    }
+    int to = s0;
+    for (int m = s0; m < s1; ++m) to += S.slot[m] < p ? 1 : 0;
+    int bc[3];
+    bin_coords(P, b % P.nbins, bc);
+    emit_sorted<T>(P, S, bc, pack_bin(P, bc), to, p);
+  }
+}
+template <typename T>
+__global__ void __launch_bounds__(SORTM_THREADS) k_sort_multi(const StepParams* __restrict__ Pp, Dev S) {
+  k_sort_multi_body<T>(Pp, S, (int)blockIdx.x);
+}
+
+// After k_sort_multi: thread t of `threads` clears its share of the bucket counts for the next
+// counting pass (the general sort clears them itself).  At the pair kernels' end, where nothing
+// waits for the stores.
+__device__ __forceinline__ void clear_counts(const StepParams& P, const Dev& S, int t, int threads) {
+  if (P.sort_range == 0 || t >= threads) return;
+  const int n = P.nbuckets;
+  for (int u = t; 4 * u < n; u += threads) {
+    if (4 * u + 3 < n) {
+      *reinterpret_cast<int4*>(S.count + 4 * u) = make_int4(0, 0, 0, 0);
+    } else {
+      for (int q = 4 * u; q < n; ++q) S.count[q] = 0;
+    }
+  }
+}
+__global__ void k_clear_counts(const StepParams* __restrict__ Pp, Dev S) {
+  clear_counts(*Pp, S, (int)(blockIdx.x * blockDim.x + threadIdx.x), (int)(gridDim.x * blockDim.x));
+}
+
+// ======================================================================================
 // Persistent bin sort (neighbour-list mode): keys, bucket scan, scatter and per-bucket sort in
 // one launch, over the same bodies as the separate kernels.  It works only on rebuild passes
 // and otherwise returns at once, so a step that keeps its list pays one launch.
@@ -475,7 +610,7 @@ __global__ void __launch_bounds__(256) k_sort_all(const StepParams* __restrict__
   const int na = P.nbuckets > 0 ? (P.nbuckets + 255) / 256 : 1;
   if (ok)
     for (int vb = blockIdx.x; vb < na; vb += (int)G)
-      k_scan_add_body(S.start, S.blocksum, P.nbuckets, S.start + P.nbuckets, vb);
+      k_scan_add_body(S.start, S.blocksum, P.nbuckets, S.start + P.nbuckets, S.count, vb);
   ok = ok && grid_barrier(sync, 3, S.err);
   if (ok)
     for (int vb = blockIdx.x; vb < np; vb += (int)G) k_scatter_body(S, vb);
@@ -807,7 +942,7 @@ __device__ inline T group_sum(T v, int lanes) {
 // spill and are slower (3D: 130 and 277 us a step against 112).
 constexpr int PAIR64_UNROLL = 4;
 template <int D, bool CT>
-__device__ inline void k_pair64_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
+__device__ inline void pair64_forces(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
   const StepParams& P = *Pp;
   const int* __restrict__ start = S.start;
   const double4* __restrict__ spos = (const double4*)S.spos;
@@ -950,11 +1085,16 @@ __device__ inline void k_pair64_body(const StepParams* __restrict__ Pp, const De
   if (sub == 0) ((double*)S.ppair)[k] = pr;
 }
 template <int D, bool CT>
+__device__ inline void k_pair64_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
+  pair64_forces<D, CT>(Pp, S, bid);
+  clear_counts(*Pp, S, bid * (int)blockDim.x + (int)threadIdx.x, S.P << Pp->pair_shift);
+}
+template <int D, bool CT>
 __global__ void __launch_bounds__(256) k_pair64(const StepParams* __restrict__ Pp, Dev S) {
   k_pair64_body<D, CT>(Pp, S, xcd_block_chunked(blockIdx.x, gridDim.x));
 }
 
-__device__ inline void k_pair_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
+__device__ inline void pair_forces(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
   const StepParams& P = *Pp;
   const int D = P.box.dim;
   const int total = S.start[P.nbuckets];
@@ -1028,6 +1168,10 @@ __device__ inline void k_pair_body(const StepParams* __restrict__ Pp, const Dev&
   float* fp = (float*)S.fpair;
   for (int dd = 0; dd < D; ++dd) fp[(size_t)dd * S.P + k] = F[dd];
   ((float*)S.ppair)[k] = pr;
+}
+__device__ inline void k_pair_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
+  pair_forces(Pp, S, bid);
+  clear_counts(*Pp, S, bid * (int)blockDim.x + (int)threadIdx.x, S.P);
 }
 // Generic FP32 kernel (pair kernel variant 1).
 __global__ void __launch_bounds__(256) k_pair(const StepParams* __restrict__ Pp, Dev S) { k_pair_body(Pp, S, xcd_block_chunked(blockIdx.x, gridDim.x)); }
@@ -1200,7 +1344,7 @@ __device__ __forceinline__ int run_coord(int sb) { return D == 3 ? (sb & 1023) :
 // At 131,071 particles (3D): 307 us with one thread per particle over single bins, 120 us with four.
 constexpr int PAIR32_UNROLL = 2;  // 4 need 98-112 VGPRs: 184 against 173 us per step
 template <int D>
-__device__ inline void k_pair32_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
+__device__ inline void pair32_forces(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
   __shared__ int guard[256][GUARD_SLOTS];  // each lane's pairs inside the LJ guard band
   const StepParams& P = *Pp;
   const float4* __restrict__ spos = (const float4*)S.spos;
@@ -1338,6 +1482,11 @@ __device__ inline void k_pair32_body(const StepParams* __restrict__ Pp, const De
   pr = P.pressure ? group_sum(pr, lanes) : 0.0f;
   if (sub == 0) ((float*)S.ppair)[k] = pr;
   if (group_sum(nguard, lanes) > GUARD_SLOTS) atomicOr(S.err, (unsigned)ERR_GUARD);
+}
+template <int D>
+__device__ inline void k_pair32_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
+  pair32_forces<D>(Pp, S, bid);
+  clear_counts(*Pp, S, bid * (int)blockDim.x + (int)threadIdx.x, S.P << Pp->pair_shift);
 }
 #define PAIR32_WPE 5  // six waves per SIMD spill
 template <int D>
@@ -2097,7 +2246,7 @@ __device__ inline void k_update_body(const StepParams* __restrict__ Pp, const De
       }
       int b = bucket_key(P, (int)p, s, xn);
       S.key[p] = b;
-      S.rank[p] = atomicAdd(&S.count[b], 1);
+      atomicAdd(&S.count[b], 1);
     } else if (emit_keys == 2) {
       list_track<D>(P, S, p, xn, sig[e], next_pass_flag(S, tsu));
     }

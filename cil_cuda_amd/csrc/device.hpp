@@ -199,6 +199,7 @@ struct StepParams {
   double rca_tt[CIL_MAX_TYPES][CIL_MAX_TYPES];    // force cut-off rc = rca*(s_p+s_q) + rcb
   double rcb_tt[CIL_MAX_TYPES][CIL_MAX_TYPES];
   double sigma_bound[CIL_MAX_TYPES];              // diameters the bins were sized for
+  int sort_range;   // buckets per workgroup of the one-launch sort (k_sort_multi); 0: general sort
   int pair_shift;   // stencil pair kernels: log2 of the lanes that share one particle
 };
 

@@ -5,8 +5,8 @@
 //   pos/vel/frc : FP64 SoA [D][P]      sigma : FP64 [P]
 //   per-cell    : FP64 / int32 [C]
 // Per-step scratch (rebuilt every step):
-//   key/rank    : int32 [P]  bin index and arrival rank (atomic counting sort)
-//   count/start : int32 [nbins(+1)]
+//   key         : int32 [P]  bin index (counting sort)
+//   count/start : int32 [nbins(+1)]  particles per bucket (then the scatter's cursors), bucket starts
 //   idx         : int32 [P]  sorted slot -> particle, ascending particle index inside a bin
 //                            (sorting network per lane, wave bitonic for large bins), so
 //                            every run is bit-reproducible
@@ -42,10 +42,10 @@ struct Dev {
   int ts_off;       // added to *ts by every reader: step offset inside a chunk of launched steps
   unsigned* err;    // [1]
   int* key;
-  int* rank;
   int* count;
   int* start;       // [nbins+1]
   int* blocksum;
+  int* slot;        // [P] k_sort_multi: a bucket's particles in arrival order
   int* idx;
   int* inv;
   void* spos;
@@ -62,8 +62,8 @@ struct Dev {
   // division / removal scratch
   int* dflag;
   int* dscan;
-  int* dblock;
-  int* nnew;        // [CIL_MAX_SPECIES]
+  unsigned* dtick;  // [1] k_div_fused: arrivals and flagged cells of the launch, zero between launches
+  int* dmark;       // [C] k_div_fused: flagged cells, zero between launches
   // neighbour-list mode
   unsigned* rebuild;  // [0..1] by the parity of a force pass's step index: nonzero = that pass
                       // re-sorts and rebuilds the list (set by the skin test, division and
