@@ -2291,6 +2291,67 @@ __global__ void k_materialize(const StepParams* __restrict__ Pp, Dev S) {
 }
 
 // ======================================================================================
+// Frames for the host: every active cell's state packed in the host views' layout, behind a header of
+// the error word and the cell counts.  One contiguous buffer means one transfer for a small colony, and
+// transfers straight into the views' order for a large one.
+// ======================================================================================
+constexpr int FRAME_HEAD = 8;           // ints: error word, CIL_MAX_SPECIES counts, padding
+constexpr int FRAME_CELL_DOUBLES = 6;   // sigma_t, pressure, theta, rho, ang_vel, rest_len
+constexpr int FRAME_CELL_INTS = 4;      // state, t0, tswitch, tpressure
+
+// Byte offsets of species arrays in the frame: per species positions, velocities, forces [n][nE][D],
+// diameters [n][nE], the cell doubles [n] each, then the cell ints [n] each (padded to 8 bytes).
+struct FrameLayout {
+  size_t vec, sig, dbl, ints, end;
+};
+__host__ __device__ inline FrameLayout frame_layout(int n, int nE, int D, size_t at) {
+  FrameLayout L;
+  L.vec = at;
+  L.sig = L.vec + (size_t)3 * n * nE * D * 8;
+  L.dbl = L.sig + (size_t)n * nE * 8;
+  L.ints = L.dbl + (size_t)FRAME_CELL_DOUBLES * n * 8;
+  L.end = L.ints + (((size_t)FRAME_CELL_INTS * n * 4 + 7) & ~(size_t)7);
+  return L;
+}
+
+__global__ void __launch_bounds__(256) k_pack_frame(const StepParams* __restrict__ Pp, Dev S, unsigned char* out) {
+  const StepParams& P = *Pp;
+  const int cslot = blockIdx.x * blockDim.x + threadIdx.x;
+  if (cslot == 0) {
+    unsigned* head = reinterpret_cast<unsigned*>(out);
+    head[0] = *S.err;
+    for (int s = 0; s < P.nspec; ++s) head[1 + s] = (unsigned)S.ncells[s];
+  }
+  if (cslot >= S.C) return;
+  int s, c;
+  if (!cell_active(P, S.ncells, cslot, &s, &c)) return;
+  const int D = P.box.dim, nE = P.nE;
+  FrameLayout L = frame_layout(S.ncells[0], nE, D, FRAME_HEAD * sizeof(int));
+  for (int q = 1; q <= s; ++q) L = frame_layout(S.ncells[q], nE, D, L.end);
+  const size_t n = (size_t)S.ncells[s];
+  double* pos = reinterpret_cast<double*>(out + L.vec);
+  double *vel = pos + n * nE * D, *frc = vel + n * nE * D;
+  double* sig = reinterpret_cast<double*>(out + L.sig);
+  for (int e = 0; e < nE; ++e) {
+    const size_t p = (size_t)cslot * nE + e, o = (size_t)c * nE + e;
+    sig[o] = S.sigma[p];
+    for (int d = 0; d < D; ++d) {
+      pos[o * D + d] = S.pos[(size_t)d * S.P + p];
+      vel[o * D + d] = S.vel[(size_t)d * S.P + p];
+      frc[o * D + d] = S.frc[(size_t)d * S.P + p];
+    }
+  }
+  double* cd = reinterpret_cast<double*>(out + L.dbl) + c;
+  const double* const src[FRAME_CELL_DOUBLES] = {S.sigma_t, S.pressure, S.theta, S.rho, S.ang_vel, S.rest_len};
+#pragma unroll
+  for (int q = 0; q < FRAME_CELL_DOUBLES; ++q) cd[(size_t)q * n] = src[q][cslot];
+  int* ci = reinterpret_cast<int*>(out + L.ints) + c;
+  const int* const isrc[FRAME_CELL_INTS] = {S.state, S.t0, S.tswitch, S.tpressure};
+#pragma unroll
+  for (int q = 0; q < FRAME_CELL_INTS; ++q) ci[(size_t)q * n] = isrc[q][cslot];
+}
+
+// ======================================================================================
 // Pair-set hook: exact FP64 law predicate over the stencil, emits UID pairs (i<j).
 // ======================================================================================
 __device__ inline int slot_to_uid_particle(const StepParams& P, const int* ncells, int pidx) {
