@@ -1506,8 +1506,10 @@ __device__ inline int list_code(int ox, int oy, int oz) { return ((ox + 4) * 9 +
 // positions stay in its own L2, and gets an equal share of each type (types differ in list
 // length).  Within an XCD the waves run type by type.  The grid holds at least
 // ceil((sum over types of ceil(waves_t / 8)) / waves per block) workgroups per XCD; waves
-// beyond an XCD's share return false.
+// beyond an XCD's share return false.  2^SH lanes share a particle.
+template <int SH>
 __device__ inline bool wave_type_slot(const StepParams& P, const Dev& S, int* tp_out, int* k_out) {
+  constexpr int PER = WAVE >> SH;
   const int lane = threadIdx.x & (WAVE - 1);
   const int x = blockIdx.x % NUM_XCD;
   const int v = __builtin_amdgcn_readfirstlane((int)(blockIdx.x / NUM_XCD) * (int)(blockDim.x / WAVE) +
@@ -1515,19 +1517,19 @@ __device__ inline bool wave_type_slot(const StepParams& P, const Dev& S, int* tp
   int tp = -1, k0 = 0, k1 = 0, acc = 0;
   for (int t = 0; t < P.ntypes; ++t) {
     const int T0 = S.start[t * P.nbins], T1 = S.start[(t + 1) * P.nbins];
-    const int nw = (T1 - T0 + WAVE - 1) / WAVE;
+    const int nw = (T1 - T0 + PER - 1) / PER;
     const int lo = (int)(((long)x * nw) / NUM_XCD), hi = (int)(((long)(x + 1) * nw) / NUM_XCD);
     if (tp < 0 && v < acc + (hi - lo)) {
       tp = t;
-      k0 = T0 + (lo + v - acc) * WAVE;
+      k0 = T0 + (lo + v - acc) * PER;
       k1 = T1;
     }
     acc += hi - lo;
   }
   if (tp < 0) return false;
   *tp_out = __builtin_amdgcn_readfirstlane(tp);
-  *k_out = k0 + lane;
-  return k0 + lane < k1;
+  *k_out = k0 + (lane >> SH);
+  return k0 + (lane >> SH) < k1;
 }
 
 // Wave-wide minimum / maximum over all 64 lanes (every lane must be active).
@@ -1554,29 +1556,35 @@ constexpr int BUILD_WIN = 160;
 // the union of their ranges fits BUILD_WIN, the wave loads it once, coalesced, into its LDS
 // window `win` and the lanes read their candidates there instead of gathering each from
 // memory.  The candidates, their order and the arithmetic are the same either way.
-template <int D>
-__device__ inline void build_list_of(const StepParams& P, const Dev& S, int tp, int k, float4* win) {
+// With 2^SH lanes per particle each lane lists the candidates whose sorted index is its own number
+// modulo 2^SH: it keeps a list of its own (lane L = k 2^SH + sub of `lanes` P 2^SH), which the pass and
+// the inner list take over.
+template <int D, int SH>
+__device__ inline void build_list_of(const StepParams& P, const Dev& S, int tp, int k, int sub, float4* win) {
   const float4* __restrict__ spos = (const float4*)S.spos;
   const int* __restrict__ start = S.start;
   const int nE = P.nE, cshift = nE - 1, spec_p = tp / nE;
   const int pidx = S.smeta[k] >> 3, cell_p = pidx >> cshift;
-  for (int d = 0; d < D; ++d) S.xref[(size_t)d * S.P + pidx] = (float)S.pos[(size_t)d * S.P + pidx];
-  S.xref[(size_t)3 * S.P + pidx] = (float)S.sigma[pidx];
+  if (SH == 0 || sub == 0) {
+    for (int d = 0; d < D; ++d) S.xref[(size_t)d * S.P + pidx] = (float)S.pos[(size_t)d * S.P + pidx];
+    S.xref[(size_t)3 * S.P + pidx] = (float)S.sigma[pidx];
+  }
   int bc[3];
   unpack_bin(P, S.sbin[k], bc);
   const float4 me = spos[k];
-  if (S.spos0) reinterpret_cast<float4*>(S.spos0)[k] = me;
+  if (S.spos0 && (SH == 0 || sub == 0)) reinterpret_cast<float4*>(S.spos0)[k] = me;
   const float wx = (float)P.w[0], wy = (float)P.w[1], wz = (float)P.w[2];
   const bool mix = P.reach[0] == 0 && P.box.pbc[0], miy = P.reach[1] == 0 && P.box.pbc[1];
   const bool miz = D == 3 && P.reach[2] == 0 && P.box.pbc[2];
   const float skin = P.skin;
-  const size_t NP = (size_t)S.P;
+  const size_t NL = (size_t)S.P << SH, L = ((size_t)k << SH) + sub;
   const int lane = threadIdx.x & (WAVE - 1);
   const bool full = __ballot(1) == ~0ull;  // all lanes present: the window can be shared
   int4* __restrict__ nl4 = (int4*)S.nl;
   const int ngroups = P.list_max >> 2;
   int slot = 0;  // next list slot; each source type starts on a group boundary
   int b0 = 0, b1 = 0, b2 = 0, b3 = 0;  // the group being filled
+  int groups = 0;  // groups of four that the particle's whole list takes
   bool over = false;
   for (int tq = 0; tq < P.ntypes; ++tq) {
     int m = 0;
@@ -1645,7 +1653,8 @@ __device__ inline void build_list_of(const StepParams& P, const Dev& S, int tp, 
               const int j1 = j1s[sg];
               int u = u0s[sg], jend = start[u + 1];
               float qz = me.z - (float)zo[sg] * wz;
-              for (int j = j0s[sg]; j < j1; ++j) {
+              const int jf = SH == 0 ? j0s[sg] : j0s[sg] + ((sub - j0s[sg]) & ((1 << SH) - 1));
+              for (int j = jf; j < j1; j += 1 << SH) {
                 while (j >= jend) {
                   ++u;
                   jend = start[u + 1];
@@ -1672,7 +1681,7 @@ __device__ inline void build_list_of(const StepParams& P, const Dev& S, int tp, 
                 ++m;
                 if (s == 3) {  // group complete: one 16-byte store
                   const int g = (slot >> 2) - 1;
-                  if (g < ngroups) nl4[(size_t)g * NP + k] = make_int4(b0, b1, b2, b3);
+                  if (g < ngroups) nl4[(size_t)g * NL + L] = make_int4(b0, b1, b2, b3);
                   else over = true;
                 }
               }
@@ -1686,14 +1695,17 @@ __device__ inline void build_list_of(const StepParams& P, const Dev& S, int tp, 
     }
     if (slot & 3) {  // partial last group of this source type (its unused slots are never read)
       const int g = slot >> 2;
-      if (g < ngroups) nl4[(size_t)g * NP + k] = make_int4(b0, b1, b2, b3);
+      if (g < ngroups) nl4[(size_t)g * NL + L] = make_int4(b0, b1, b2, b3);
       else over = true;
       slot = (slot + 3) & ~3;
     }
-    S.nlt[(size_t)tq * NP + k] = m;
+    S.nlt[(size_t)tq * NL + L] = m;
+    if (SH > 0) groups += (group_sum(m, 1 << SH) + 3) >> 2;
   }
+  // the capacity is the particle's, whatever number of lanes shares its list
+  if (SH > 0) over = group_sum(over || groups > ngroups ? 1 : 0, 1 << SH) > 0;
   if (over) {  // capacity error: an empty list keeps the pair loop inside the allocation
-    for (int tq = 0; tq < P.ntypes; ++tq) S.nlt[(size_t)tq * NP + k] = 0;
+    for (int tq = 0; tq < P.ntypes; ++tq) S.nlt[(size_t)tq * NL + L] = 0;
     atomicOr(S.err, (unsigned)ERR_LIST);
   }
 }
@@ -1772,7 +1784,7 @@ __device__ __forceinline__ int4 list_group(const char* __restrict__ nlb, unsigne
 // starts on a group boundary, as in the list build.
 struct InnerList {
   int4* nl4;
-  size_t NP;
+  size_t NP;  // lanes' lists, and this lane's
   int k, ngroups;
   float rca, rcb, skin;  // the list radius of the current source type: (rca (s_i + s_j) + rcb + skin) 1.001
   int slot, m, b0, b1, b2, b3;
@@ -1806,7 +1818,7 @@ struct InnerList {
 
 template <int D, int LC, bool MI, bool SH, bool RF>
 __device__ __forceinline__ void list_segment(const StepParams& P, const Dev& S, const Law32& Lw, const float4* tab,
-                                             const float4& me, int k, int pidx, uint32_t ts, float cadh, int n,
+                                             const float4& me, int* gslot, int pidx, uint32_t ts, float cadh, int n,
                                              const char* __restrict__ nlb, unsigned& off, unsigned stride, float& Fx,
                                              float& Fy, float& Fz, float& pr, int& nguard, InnerList& il) {
   const float4* __restrict__ spos = (const float4*)S.spos;
@@ -1829,7 +1841,7 @@ __device__ __forceinline__ void list_segment(const StepParams& P, const Dev& S, 
       bool guard;
       f0 = lj_term32<SH>(Lw, r.w + me.w, r2, &guard);
       if (guard) {  // rare: recorded for the exact FP64 decision after the loop
-        if (nguard < GUARD_SLOTS) S.gslot[(size_t)k * GUARD_SLOTS + nguard] = (int)(e >> 10);
+        if (nguard < GUARD_SLOTS) gslot[nguard] = (int)(e >> 10);
         ++nguard;
       }
     } else if (LC == CIL_LAW_SC) {
@@ -1891,7 +1903,7 @@ __device__ __forceinline__ void list_segment(const StepParams& P, const Dev& S, 
 // this pass's rebuild flag is set.  Same law code, exclusions, guard band and per-type wave
 // layout as k_pair32.  List groups are addressed with 32-bit byte offsets
 // (list_max * P * 4 < 2^32, checked by the host).
-template <int D>
+template <int D, int SH>
 __device__ inline void k_pair_list_body(const StepParams* __restrict__ Pp, const Dev& S) {
   const StepParams& P = *Pp;
   __shared__ float4 tab[LIST_CODES];
@@ -1903,8 +1915,9 @@ __device__ inline void k_pair_list_body(const StepParams* __restrict__ Pp, const
   if (rebuild && (__hip_atomic_load(S.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERR_SYNC)) return;
   if (rebuild && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(S.rebuild + 2, 1u);  // list epoch
   int tp, k;
-  if (!wave_type_slot(P, S, &tp, &k)) return;
-  if (rebuild) build_list_of<D>(P, S, tp, k, bwin[threadIdx.x / WAVE]);
+  if (!wave_type_slot<SH>(P, S, &tp, &k)) return;
+  const int sub = SH == 0 ? 0 : (int)(threadIdx.x & ((1 << SH) - 1));
+  if (rebuild) build_list_of<D, SH>(P, S, tp, k, sub, bwin[threadIdx.x / WAVE]);
   const float4* __restrict__ spos = (const float4*)S.spos;
   const uint32_t ts = (uint32_t)step_ts(S);
   const int nE = P.nE, spec_p = tp / nE;
@@ -1913,9 +1926,10 @@ __device__ inline void k_pair_list_body(const StepParams* __restrict__ Pp, const
   const float4 me = spos[k];
   const bool mi = (P.reach[0] == 0 && P.box.pbc[0]) || (P.reach[1] == 0 && P.box.pbc[1]) ||
                   (D == 3 && P.reach[2] == 0 && P.box.pbc[2]);
-  const size_t NP = (size_t)S.P;
-  const unsigned stride = 16u * (unsigned)S.P;
-  unsigned off = 16u * (unsigned)k;
+  const size_t NP = (size_t)S.P, NL = NP << SH, L = ((size_t)k << SH) + sub;  // lanes' lists, this lane's
+  const unsigned stride = 16u * (unsigned)NL;
+  unsigned off = 16u * (unsigned)L;
+  int* const gslot = S.gslot + L * GUARD_SLOTS;
   float Fx = 0.f, Fy = 0.f, Fz = 0.f, pr = 0.f;
   int nguard = 0;
   // two-level lists: a refresh pass evaluates the outer list and writes the inner one; other
@@ -1928,9 +1942,9 @@ __device__ inline void k_pair_list_body(const StepParams* __restrict__ Pp, const
     const bool inner = two && !RF;
     const char* __restrict__ nlb = inner ? (const char*)S.nl_in : (const char*)S.nl;
     const int* __restrict__ nlt = inner ? S.nlt_in : S.nlt;
-    InnerList il{(int4*)S.nl_in, NP, k, P.list_max >> 2, 0.f, 0.f, P.skin_in, 0, 0, 0, 0, 0, 0, false};
+    InnerList il{(int4*)S.nl_in, NL, (int)L, P.list_max >> 2, 0.f, 0.f, P.skin_in, 0, 0, 0, 0, 0, 0, false};
     for (int tq = 0; tq < P.ntypes; ++tq) {
-      const int n = nlt[(size_t)tq * NP + k];
+      const int n = nlt[(size_t)tq * NL + L];
       if (n > 0) {
         const Law32 Lw = law32(P, tp, tq);
         const float cadh = (tq / nE == spec_p) ? 1.0f : ca_p;  // scale for f0 >= 0 (MD.cu:345-360)
@@ -1939,7 +1953,7 @@ __device__ inline void k_pair_list_body(const StepParams* __restrict__ Pp, const
           il.rcb = (float)P.rcb_tt[tp][tq];
         }
 #define CIL_SEG(LC, MIV, SHV)                                                                                 \
-  list_segment<D, LC, MIV, SHV, RF>(P, S, Lw, tab, me, k, pidx, ts, cadh, n, nlb, off, stride, Fx, Fy, Fz, pr, \
+  list_segment<D, LC, MIV, SHV, RF>(P, S, Lw, tab, me, gslot, pidx, ts, cadh, n, nlb, off, stride, Fx, Fy, Fz, pr, \
                                     nguard, il)
         if (Lw.law == CIL_LAW_LJ) {
           if (Lw.shifted) {
@@ -1958,24 +1972,34 @@ __device__ inline void k_pair_list_body(const StepParams* __restrict__ Pp, const
         }
 #undef CIL_SEG
       }
-      if (RF) il.end_type(S.nlt_in + (size_t)tq * NP + k);
+      if (RF) il.end_type(S.nlt_in + (size_t)tq * NL + L);
     }
     if (RF) {
       if (il.over) {  // capacity error: an empty inner list keeps later passes inside the allocation
-        for (int tq = 0; tq < P.ntypes; ++tq) S.nlt_in[(size_t)tq * NP + k] = 0;
+        for (int tq = 0; tq < P.ntypes; ++tq) S.nlt_in[(size_t)tq * NL + L] = 0;
         atomicOr(S.err, (unsigned)ERR_LIST);
       }
-      for (int d = 0; d < D; ++d) S.xref_in[(size_t)d * NP + pidx] = (float)S.pos[(size_t)d * NP + pidx];
+      if (SH == 0 || sub == 0)
+        for (int d = 0; d < D; ++d) S.xref_in[(size_t)d * NP + pidx] = (float)S.pos[(size_t)d * NP + pidx];
     }
   };
   if (refresh) run_types(std::true_type{});
   else run_types(std::false_type{});
   if (nguard > 0) {
     float g[3] = {0.f, 0.f, 0.f};
-    guard_force(P, S, k, S.gslot + (size_t)k * GUARD_SLOTS, nguard, g);
+    guard_force(P, S, k, gslot, nguard, g);
     Fx += g[0];
     Fy += g[1];
     if (D == 3) Fz += g[2];
+  }
+  if (SH > 0) {
+    constexpr int lanes = 1 << SH;
+    Fx = group_sum(Fx, lanes);
+    Fy = group_sum(Fy, lanes);
+    if (D == 3) Fz = group_sum(Fz, lanes);
+    if (P.pressure) pr = group_sum(pr, lanes);
+    nguard = group_sum(nguard, lanes);
+    if (sub != 0) return;
   }
   float* fp = (float*)S.fpair;
   fp[k] = Fx;
@@ -1984,10 +2008,10 @@ __device__ inline void k_pair_list_body(const StepParams* __restrict__ Pp, const
   ((float*)S.ppair)[k] = P.pressure ? pr : 0.0f;
   if (nguard > GUARD_SLOTS) atomicOr(S.err, (unsigned)ERR_GUARD);
 }
-template <int D>
+template <int D, int SH>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LIST_WAVES_PER_EU)))
 k_pair_list(const StepParams* __restrict__ Pp, Dev S) {
-  k_pair_list_body<D>(Pp, S);
+  k_pair_list_body<D, SH>(Pp, S);
 }
 
 // Both rebuild flags (either step parity) to v.

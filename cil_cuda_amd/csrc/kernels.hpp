@@ -51,8 +51,8 @@ struct Dev {
   void* spos;
   int* smeta;
   int* sbin;        // bin of each sorted particle, packed coordinates (pack_bin)
-  int* gslot;       // [P][4] FP32 LJ pairs inside the cut-off guard band (sorted source index),
-                    // resolved in FP64 by the pair kernel itself after its pair loop
+  int* gslot;       // list mode: [lists][4] FP32 LJ pairs inside the cut-off guard band (sorted source
+                    // index), resolved in FP64 by the pair kernel itself after its pair loop
   void* fpair;
   void* ppair;
   const double* ext;
@@ -69,9 +69,10 @@ struct Dev {
                       // re-sorts and rebuilds the list (set by the skin test, division and
                       // host-initiated sorts; the update of step u clears word u & 1, whose
                       // pass has run); [2] list epoch, counts the builds
-  int* nl;            // [list_max / 4][P][4] groups of (sorted index << 10 | bin offset code);
-                      // each source type starts on a group boundary
-  int* nlt;           // [ntypes][P] entries per source type
+  int* nl;            // [list_max / 4][lists][4] groups of (sorted index << 10 | bin offset code); each
+                      // source type starts on a group boundary; one list per lane of a particle,
+                      // lists = P lanes
+  int* nlt;           // [ntypes][lists] entries per source type
   float* xref;        // [4][P] positions (x, y, z) and diameter at the last build (particle order)
   float* spos0;       // [P][4] or null: the sorted bin-local positions and diameter at the last
                       // build (sorted order), kept for the surrogate's kNN candidate lists
@@ -79,8 +80,8 @@ struct Dev {
   // cut-off + inner skin at its last refresh, in the same order; a pass refreshes it, while
   // evaluating the outer list, when the outer list was rebuilt or a particle has moved more
   // than inner skin / 2 since the refresh (flags rebuild[4..5], by parity like [0..1])
-  int* nl_in;         // [list_max / 4][P][4], the layout of nl
-  int* nlt_in;        // [ntypes][P]
+  int* nl_in;         // [list_max / 4][lists][4], the layout of nl
+  int* nlt_in;        // [ntypes][lists]
   float* xref_in;     // [3][P] positions at the last refresh (particle order)
   // integrator: 0 Euler (one force pass per step, at step index f); 1 stochastic Heun (two
   // passes per step: the corrector's at the step's own index with phase 1, the final one at the

@@ -1,4 +1,4 @@
-"""The stencil pair kernels with every number of lanes per particle, against the CPU oracle.
+"""The pair kernels with every number of lanes per particle, against the CPU oracle.
 
 The lanes per particle follow the context's particle slots, so a large capacity puts a small colony
 on the path of a large one.  Colonies: one particle, a partial last wave in each type, a box of one
@@ -39,7 +39,7 @@ def _colony(dim, n, L, periodic, law, capacity, seed, stray=0):
     return p, box, col
 
 
-def _worst(p, box, col, tol, floor):
+def _worst(p, box, col, tol, floor, skin=0.0):
     dim = p.dim
     q = abi.Params.from_buffer_copy(p)
     q.precision = abi.PREC_FP64
@@ -50,6 +50,8 @@ def _worst(p, box, col, tol, floor):
     orc.close()
     md = HipMD(p, box, [sp["capacity"] for sp in col.species])
     md.upload(col)
+    if skin:
+        md.set_neighbour_list(True, skin, 1024)
     frc, pr = md.forces()
     md.close()
     fref = ref.flat("frc").reshape(-1, dim)
@@ -86,3 +88,52 @@ def test_pair_lanes_fp32(gpu, dim, cap, law):
         # bins (up to 1.3 wide), 2^-22 for discs up to 3 outside them
         worst, _, _ = _worst(p, box, col, 1e-5, 0.02 if stray else 0.01)
         assert worst <= 1.0, (n, L, periodic, worst)
+
+
+LIST_CAPS = (400, 20000, 100000, 300000)  # eight, four, two and one lane per particle in 3D
+
+
+@pytest.mark.parametrize("law", [abi.LAW_SC, abi.LAW_HZ])
+@pytest.mark.parametrize("cap", LIST_CAPS)
+def test_list_lanes(gpu, cap, law):
+    for n, L, periodic, stray in CASES:
+        p, box, col = _colony(3, n, L, periodic, law, cap, seed=100 + n + law)
+        p.precision = abi.PREC_FP32
+        worst, _, _ = _worst(p, box, col, 1e-5, 0.01, skin=0.3)
+        assert worst <= 1.0, (n, L, periodic, worst)
+
+
+@pytest.mark.parametrize("cap", LIST_CAPS)
+def test_two_level_list_lanes(gpu, cap):
+    """The inner list keeps each lane's entries and their order: bit-identical to one level, through
+    refreshes and rebuilds; and the capacity is the particle's, whatever the lanes."""
+    p, box, col = configs.relaxed_bulk_3d(4096, seed=3, precision=abi.PREC_FP32)
+    ends = []
+    for inner in (0.0, 0.05):
+        md = HipMD(p, box, [cap + sp["capacity"] for sp in col.species])
+        md.upload(col)
+        md.set_neighbour_list(True, 0.15, 160, inner_skin=inner)
+        md.forces(want=False)
+        md.step(150, 0)
+        c = col.copy()
+        md.download(c)
+        md.close()
+        ends.append(c)
+    for f in ("pos", "vel", "frc"):
+        assert np.array_equal(ends[0].flat(f), ends[1].flat(f)), f
+    codes = []
+    for slots in (48, 52, 56, 60, 64, 68, 72, 76, 80, 84, 88, 92, 96, 100, 104, 108, 112, 116, 120):
+        md = HipMD(p, box, [cap + sp["capacity"] for sp in col.species])
+        md.upload(col)
+        md.set_neighbour_list(True, 0.15, slots)
+        try:
+            md.forces(want=False)
+            codes.append(slots)
+        except abi.CilError as e:
+            assert e.code == -3
+        md.close()
+    _SMALLEST.setdefault("slots", codes[0])
+    assert codes[0] == _SMALLEST["slots"] and codes == list(range(codes[0], 121, 4))
+
+
+_SMALLEST = {}
