@@ -481,15 +481,16 @@ __device__ inline void k_sort_multi_body(const StepParams* __restrict__ Pp, cons
   }
   __syncthreads();
   // this range's particles, in arrival order inside a bucket
-  for (int p0 = 0; p0 < S.P; p0 += 4 * SORTM_THREADS) {
-    int b[4];
+  constexpr int KEYS = 8;  // in flight per thread
+  for (int p0 = 0; p0 < S.P; p0 += KEYS * SORTM_THREADS) {
+    int b[KEYS];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < KEYS; ++q) {
       const int p = p0 + q * SORTM_THREADS + tid;
       b[q] = p < S.P ? S.key[p] : -1;
     }
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < KEYS; ++q) {
       if (b[q] < lo || b[q] >= hi) continue;
       const int l = b[q] - lo;
       S.slot[st[l] + atomicAdd(&cur[l], 1)] = p0 + q * SORTM_THREADS + tid;
@@ -1081,8 +1082,10 @@ __device__ inline void pair64_forces(const StepParams* __restrict__ Pp, const De
     const double f = group_sum(F[d], lanes);
     if (sub == 0) fp[(size_t)d * S.P + k] = f;
   }
-  if (CT && P.pressure) pr = group_sum(pr, lanes);
-  if (sub == 0) ((double*)S.ppair)[k] = pr;
+  if (P.pressure) {  // read back under the same condition only
+    if (CT) pr = group_sum(pr, lanes);
+    if (sub == 0) ((double*)S.ppair)[k] = pr;
+  }
 }
 template <int D, bool CT>
 __device__ inline void k_pair64_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
@@ -1479,8 +1482,10 @@ __device__ inline void pair32_forces(const StepParams* __restrict__ Pp, const De
     const float f = group_sum(F[d], lanes);
     if (sub == 0) fp[(size_t)d * S.P + k] = f;
   }
-  pr = P.pressure ? group_sum(pr, lanes) : 0.0f;
-  if (sub == 0) ((float*)S.ppair)[k] = pr;
+  if (P.pressure) {
+    pr = group_sum(pr, lanes);
+    if (sub == 0) ((float*)S.ppair)[k] = pr;
+  }
   if (group_sum(nguard, lanes) > GUARD_SLOTS) atomicOr(S.err, (unsigned)ERR_GUARD);
 }
 template <int D>
@@ -2005,7 +2010,7 @@ __device__ inline void k_pair_list_body(const StepParams* __restrict__ Pp, const
   fp[k] = Fx;
   fp[NP + k] = Fy;
   if (D == 3) fp[2 * NP + k] = Fz;
-  ((float*)S.ppair)[k] = P.pressure ? pr : 0.0f;
+  if (P.pressure) ((float*)S.ppair)[k] = pr;
   if (nguard > GUARD_SLOTS) atomicOr(S.err, (unsigned)ERR_GUARD);
 }
 template <int D, int SH>
@@ -2024,7 +2029,9 @@ __global__ void k_set_flags(unsigned* flag, unsigned v, unsigned vin) {
 
 
 // ======================================================================================
-// Noise draws (updateWienerProcess, CIL.cu:793-818), reference noise modes only.
+// Noise draws (updateWienerProcess, CIL.cu:793-818) into the noise arrays, reference noise modes only:
+// external deviates, and counter draws where the cell forces do not make them themselves (batches, and
+// a pass whose step index the caller then changes).
 // ======================================================================================
 __device__ inline void k_noise_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
   const StepParams& P = *Pp;
@@ -2052,25 +2059,20 @@ __device__ inline void k_noise_body(const StepParams* __restrict__ Pp, const Dev
     }
   }
   if (P.noise == CIL_NOISE_CELL_WIENER) {
-    for (int d = 0; d < D; ++d) {
-      double w = 0.0;
-      if (sp.d_noise > 0.0) {
-        double z;
-        long at = off_passive + (long)c * D + d;
-        if (blk && at >= S.ext_per_step) {
+    double W[3];
+    if (blk) {
+      for (int d = 0; d < D; ++d) {
+        const long at = off_passive + (long)c * D + d;
+        if (sp.d_noise > 0.0 && at >= S.ext_per_step) {
           atomicOr(S.err, (unsigned)ERR_NOISE);
           return;
         }
-        if (blk) z = blk[at];
-        else {
-          double zz[2];
-          philox_normal2(P.seed, cell_key(s, c), (uint32_t)ts, force_stream(S, ST_WIENER), (uint32_t)(d >> 1), zz);
-          z = zz[d & 1];
-        }
-        w = sp.d_noise * z;
+        W[d] = sp.d_noise > 0.0 ? sp.d_noise * blk[at] : 0.0;
       }
-      S.wiener[(size_t)cslot * 3 + d] = w;
+    } else {
+      counter_wiener(P, S, s, c, ts, D, W);
     }
+    for (int d = 0; d < D; ++d) S.wiener[(size_t)cslot * 3 + d] = W[d];
   }
   if (P.active_noise && P.nE == 2) {
     long ar = off_active, aa = off_active;
@@ -2084,15 +2086,17 @@ __device__ inline void k_noise_body(const StepParams* __restrict__ Pp, const Dev
       for (int k = 0; k < s; ++k)
         if (P.sp[k].d_noise_angular > 0.0) aa += S.ncells[k];
     }
-    double zz[2] = {0, 0};
     if (blk && (ar + c >= S.ext_per_step || aa + c >= S.ext_per_step)) {
       atomicOr(S.err, (unsigned)ERR_NOISE);
       return;
     }
-    if (!blk) philox_normal2(P.seed, cell_key(s, c), (uint32_t)ts, force_stream(S, ST_ACTIVE), 0, zz);
     double wr = 0, wa = 0;
-    if (sp.d_noise_radial > 0.0) wr = sp.d_noise_radial * (blk ? blk[ar + c] : zz[0]);
-    if (sp.d_noise_angular > 0.0) wa = sp.d_noise_angular * (blk ? blk[aa + c] : zz[1]);
+    if (blk) {
+      if (sp.d_noise_radial > 0.0) wr = sp.d_noise_radial * blk[ar + c];
+      if (sp.d_noise_angular > 0.0) wa = sp.d_noise_angular * blk[aa + c];
+    } else {
+      counter_active(P, S, s, c, ts, &wr, &wa);
+    }
     S.awiener[(size_t)cslot * 2] = wr;
     S.awiener[(size_t)cslot * 2 + 1] = wa;
   }
@@ -2102,7 +2106,7 @@ __global__ void k_noise(const StepParams* __restrict__ Pp, Dev S) { k_noise_body
 // ======================================================================================
 // Forces of one cell at the last force evaluation: intra (lazy) + pair (sorted).
 // ======================================================================================
-template <typename T, int DIM, int NE>
+template <typename T, int DIM, int NE, bool DRAW>
 __device__ inline void cell_total_force(const StepParams& P, const Dev& S, int s, int c, int cslot, bool materialized,
                                         double pos[2][3], double vel[2][3], const double* sig, double F[2][3],
                                         double* pc, bool* pos1_changed) {
@@ -2114,7 +2118,7 @@ __device__ inline void cell_total_force(const StepParams& P, const Dev& S, int s
     *pc = S.pressure[cslot];
     return;
   }
-  intra_cell<DIM, NE>(P, S, s, c, cslot, step_ts(S), pos, vel, sig, F, pos1_changed);
+  intra_cell<DIM, NE, DRAW>(P, S, s, c, cslot, step_ts(S), pos, vel, sig, F, pos1_changed);
   const T* fp = (const T*)S.fpair;
   double pr = 0.0;
   for (int e = 0; e < nE; ++e) {
@@ -2178,8 +2182,12 @@ __device__ inline void list_track(const StepParams& P, const Dev& S, size_t p, c
   }
 }
 
-template <typename T, int DIM, int NE>
-__device__ inline void k_update_body(const StepParams* __restrict__ Pp, const Dev& S, int materialized, int emit_keys, int bid) {
+// flags: forces are the materialised ones; a step inside a chunk of launched steps, whose velocities the
+// next step replaces unread (they are stored only where the intra force reads them).
+constexpr int UPD_MATERIALIZED = 1, UPD_MID_CHUNK = 4;
+constexpr int UPD_STORED_NOISE = 2;  // host only: the kernel that reads the pass's noise from the arrays
+template <typename T, int DIM, int NE, bool DRAW>
+__device__ inline void k_update_body(const StepParams* __restrict__ Pp, const Dev& S, int flags, int emit_keys, int bid) {
   const StepParams& P = *Pp;
   // list mode: the flag of the previous force pass (same step parity as this update) has been
   // used; the skin test below sets the other one, for this step's force pass
@@ -2211,8 +2219,10 @@ __device__ inline void k_update_body(const StepParams* __restrict__ Pp, const De
   }
   double pc;
   bool pos1_changed;
-  cell_total_force<T, DIM, NE>(P, S, s, c, cslot, materialized != 0, pos, vel, sig, F, &pc, &pos1_changed);
+  const bool materialized = flags & UPD_MATERIALIZED;
+  cell_total_force<T, DIM, NE, DRAW>(P, S, s, c, cslot, materialized, pos, vel, sig, F, &pc, &pos1_changed);
   if (!materialized && P.pressure) S.pressure[cslot] = pc;
+  const bool keep_vel = !(flags & UPD_MID_CHUNK) || need_vel;
   const int tsu = step_ts(S);  // step index before the increment (FDT noise key)
   double area = sigma2area(sig[0]);
   double pND = pc / sp.cycle_p0;
@@ -2258,8 +2268,11 @@ __device__ inline void k_update_body(const StepParams* __restrict__ Pp, const De
       S.pos[(size_t)d * S.P + p] = xn[d];
       // Heun leaves the velocities alone, except for the zero-velocity kick of a single disc
       // (MD.cu:609-614), which the reference writes into the velocity array
-      if (!S.heun) S.vel[(size_t)d * S.P + p] = F[e][d] * mu;
-      else if (nE == 1 && need_vel) S.vel[(size_t)d * S.P + p] = vel[e][d];
+      if (!S.heun) {
+        if (keep_vel) S.vel[(size_t)d * S.P + p] = F[e][d] * mu;
+      } else if (nE == 1 && need_vel) {
+        S.vel[(size_t)d * S.P + p] = vel[e][d];
+      }
     }
     if (emit_keys == 1) {
       bool finite = true;
@@ -2278,15 +2291,14 @@ __device__ inline void k_update_body(const StepParams* __restrict__ Pp, const De
 }
 // Register budget: six waves per SIMD for single-disc cells (no spills); two-disc cells keep
 // the compiler's own allocation.
-template <typename T, int DIM, int NE>
+template <typename T, int DIM, int NE, bool DRAW>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NE == 1 ? 6 : 1)))
-k_update(const StepParams* __restrict__ Pp, Dev S, int materialized,
-                                                int emit_keys) {
-  k_update_body<T, DIM, NE>(Pp, S, materialized, emit_keys, (int)blockIdx.x);
+k_update(const StepParams* __restrict__ Pp, Dev S, int flags, int emit_keys) {
+  k_update_body<T, DIM, NE, DRAW>(Pp, S, flags, emit_keys, (int)blockIdx.x);
 }
 
 // Forces at the current state into the canonical FP64 frc array (for download / parity).
-template <typename T, int DIM, int NE>
+template <typename T, int DIM, int NE, bool DRAW>
 __global__ void k_materialize(const StepParams* __restrict__ Pp, Dev S) {
   const StepParams& P = *Pp;
   int cslot = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2304,7 +2316,7 @@ __global__ void k_materialize(const StepParams* __restrict__ Pp, Dev S) {
     }
   }
   bool pos1_changed;
-  cell_total_force<T, DIM, NE>(P, S, s, c, cslot, false, pos, vel, sig, F, &pc, &pos1_changed);
+  cell_total_force<T, DIM, NE, DRAW>(P, S, s, c, cslot, false, pos, vel, sig, F, &pc, &pos1_changed);
   for (int e = 0; e < nE; ++e)
     for (int d = 0; d < D; ++d) S.frc[(size_t)d * S.P + (size_t)cslot * nE + e] = F[e][d];
   if (pos1_changed)

@@ -199,9 +199,30 @@ __device__ inline void on_sphere_counter(uint64_t seed, uint32_t id, uint32_t ts
   for (int d = 0; d < D; ++d) n[d] *= norm;
 }
 
+// Noise of cell (s, c) at force pass index ts (updateWienerProcess, CIL.cu:793-818) from the counter
+// streams: the passive vector, and the radial and angular active amplitudes.
+__device__ inline void counter_wiener(const StepParams& P, const Dev& S, int s, int c, int ts, int D, double* W) {
+  const cil_species& sp = P.sp[s];
+  double zz[4] = {0.0, 0.0, 0.0, 0.0};
+  if (sp.d_noise > 0.0)
+    for (int k = 0; 2 * k < D; ++k)
+      philox_normal2(P.seed, cell_key(s, c), (uint32_t)ts, force_stream(S, ST_WIENER), (uint32_t)k, zz + 2 * k);
+  for (int d = 0; d < D; ++d) W[d] = sp.d_noise > 0.0 ? sp.d_noise * zz[d] : 0.0;
+}
+__device__ inline void counter_active(const StepParams& P, const Dev& S, int s, int c, int ts, double* Wr, double* Wt) {
+  const cil_species& sp = P.sp[s];
+  double zz[2];
+  philox_normal2(P.seed, cell_key(s, c), (uint32_t)ts, force_stream(S, ST_ACTIVE), 0, zz);
+  *Wr = sp.d_noise_radial > 0.0 ? sp.d_noise_radial * zz[0] : 0.0;
+  *Wt = sp.d_noise_angular > 0.0 ? sp.d_noise_angular * zz[1] : 0.0;
+}
+
 // DIM, NE: box dimension and discs per cell (compile-time, so the per-disc arrays stay in
 // registers); they must equal P.box.dim and P.nE.
-template <int DIM, int NE>
+// DRAW: reference noise of the counter streams is drawn here, from the pass's index; otherwise it is read
+// from the arrays that the pass filled.  (Compile-time: the draws' registers would spill in the kernels
+// of colonies without such noise, 39 -> 45 us per update at 1,048,576 particles.)
+template <int DIM, int NE, bool DRAW>
 __device__ inline void intra_cell(const StepParams& P, const Dev& S, int s, int c, int cslot, int ts,
                                   double pos[2][3], double vel[2][3], const double* sig, double F[2][3],
                                   bool* pos1_changed) {
@@ -255,7 +276,13 @@ __device__ inline void intra_cell(const StepParams& P, const Dev& S, int s, int 
       }
     }
     if (P.active_noise && D == 2) {
-      double Wr = S.awiener[(size_t)cslot * 2], Wt = S.awiener[(size_t)cslot * 2 + 1];
+      double Wr, Wt;
+      if (!DRAW) {
+        Wr = S.awiener[(size_t)cslot * 2];
+        Wt = S.awiener[(size_t)cslot * 2 + 1];
+      } else {
+        counter_active(P, S, s, c, ts, &Wr, &Wt);
+      }
       rnd[0] = 0.5 * (Wr * rij[0] / r - Wt * rij[1]);
       rnd[1] = 0.5 * (Wr * rij[1] / r + Wt * rij[0]);
     }
@@ -289,9 +316,15 @@ __device__ inline void intra_cell(const StepParams& P, const Dev& S, int s, int 
   }
   for (int e = 0; e < nE; ++e)
     for (int k = 0; k < P.nwalls; ++k) flat_wall(P.walls[k], sig[e], pos[e], F[e]);
-  if (P.noise == CIL_NOISE_CELL_WIENER)
+  if (P.noise == CIL_NOISE_CELL_WIENER) {
+    double W[3];
+    if (!DRAW)
+      for (int d = 0; d < D; ++d) W[d] = S.wiener[(size_t)cslot * 3 + d];
+    else
+      counter_wiener(P, S, s, c, ts, D, W);
     for (int e = 0; e < nE; ++e)
-      for (int d = 0; d < D; ++d) F[e][d] += sp.zeta[e] * S.wiener[(size_t)cslot * 3 + d];
+      for (int d = 0; d < D; ++d) F[e][d] += sp.zeta[e] * W[d];
+  }
 }
 
 }  // namespace cil
