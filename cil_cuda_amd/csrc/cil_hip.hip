@@ -282,10 +282,10 @@ __device__ inline void emit_sorted(const StepParams& P, const Dev& S, const int*
   const int cslot = p / P.nE, e = p - cslot * P.nE;
   const int sp = species_of_cell(P, cslot);
   const int t = sp * P.nE + e;
-  S.smeta[k] = p * 8 + t;
+  S.smeta[k] = p * 8 + P.cls[t];
   S.sbin[k] = pb;
   S.inv[p] = k;
-  if (S.sigma[p] > P.sigma_bound[t]) atomicOr(S.err, (unsigned)ERR_CUTOFF);
+  if (S.sigma[p] > P.sigma_elem[t]) atomicOr(S.err, (unsigned)ERR_CUTOFF);
   write_sorted<T>(P, S, bc, k, p);
 }
 
@@ -313,8 +313,31 @@ __device__ inline void binsort_bucket_wave(const StepParams& P, const Dev& S, in
     if (lane < n) emit_sorted<T>(P, S, bc, pb, s0 + lane, v);
     return;
   }
-  if (n > BINSORT_MAX) {
+  if (n > P.nE * BINSORT_MAX) {
     if (lane == 0) atomicOr(S.err, (unsigned)ERR_BIN_OVERFLOW);
+    return;
+  }
+  if (n > BINSORT_MAX) {  // a class of two element types (each within the limit): places by counting
+    int odd = 0;
+    for (int i = lane; i < n; i += WAVE) {
+      const int p = S.idx[s0 + i];
+      S.slot[s0 + i] = p;
+      odd += p & 1;
+    }
+#pragma unroll
+    for (int o = WAVE / 2; o > 0; o >>= 1) odd += __shfl_xor(odd, o, WAVE);
+    if (P.nE == 1 || odd > BINSORT_MAX || n - odd > BINSORT_MAX) {
+      if (lane == 0) atomicOr(S.err, (unsigned)ERR_BIN_OVERFLOW);
+      return;
+    }
+    __threadfence_block();
+    __builtin_amdgcn_wave_barrier();
+    for (int i = lane; i < n; i += WAVE) {
+      const int p = S.slot[s0 + i];
+      int to = s0;
+      for (int m = 0; m < n; ++m) to += S.slot[s0 + m] < p ? 1 : 0;
+      emit_sorted<T>(P, S, bc, pb, to, p);
+    }
     return;
   }
   // One wave sorts its own LDS region; only wave-local ordering is needed between stages
@@ -501,12 +524,18 @@ __device__ inline void k_sort_multi_body(const StepParams* __restrict__ Pp, cons
   for (int k = st[0] + tid; k < end; k += SORTM_THREADS) {
     const int p = S.slot[k], b = S.key[p], l = b - lo;
     const int s0 = st[l], s1 = st[l + 1];
-    if (s1 - s0 > BINSORT_MAX) {
+    if (s1 - s0 > P.nE * BINSORT_MAX) {
       if (k == s0) atomicOr(S.err, (unsigned)ERR_BIN_OVERFLOW);
       continue;
     }
     int to = s0;
     for (int m = s0; m < s1; ++m) to += S.slot[m] < p ? 1 : 0;
+    if (s1 - s0 > BINSORT_MAX && k == s0) {  // a class of two element types: the limit holds for each
+      int odd = 0;
+      for (int m = s0; m < s1; ++m) odd += S.slot[m] & 1;
+      if (P.nE == 1 || odd > BINSORT_MAX || s1 - s0 - odd > BINSORT_MAX)
+        atomicOr(S.err, (unsigned)ERR_BIN_OVERFLOW);
+    }
     int bc[3];
     bin_coords(P, b % P.nbins, bc);
     emit_sorted<T>(P, S, bc, pack_bin(P, bc), to, p);
@@ -957,7 +986,7 @@ __device__ inline void pair64_forces(const StepParams* __restrict__ Pp, const De
   if (k >= k1) return;
   const uint32_t ts = (uint32_t)step_ts(S);
   const int nE = P.nE, cshift = nE - 1;  // cell = particle >> cshift (nE is 1 or 2)
-  const int spec_p = tp / nE;
+  const int spec_p = P.cls_spec[tp];
   const int pidx = smeta[k] >> 3, cell_p = pidx >> cshift;
   const double4 me = spos[k];
   int bc[3];
@@ -980,7 +1009,7 @@ __device__ inline void pair64_forces(const StepParams* __restrict__ Pp, const De
     if (Rx < 0) continue;
     const int Rm = D == 3 ? P.reach_tt[tp][tq][1] : 0, Rr = P.reach_tt[tp][tq][D - 1];
     const PairLaw E = load_law(P, tp, tq);
-    const int spec_q = tq / nE;
+    const int spec_q = P.cls_spec[tq];
     const double rca = P.rca_tt[tp][tq], rcb = P.rcb_tt[tp][tq];
     const float rcp = fmaf((float)rca, (float)(me.w + P.sigma_bound[tq]), (float)rcb) * 1.001f + 1e-6f;
     const float rcp2 = rcp * rcp;
@@ -1331,7 +1360,7 @@ __device__ inline void guard_force(const StepParams& P, const Dev& S, int k, con
     float f = (s6 - 2.0f * s6 * s6) * ir2;
     if (P.force_shifted) f -= lj_f0(sij2, rc2) * sqrtf(rc2 * ir2);
     float f0 = f * (float)A.eps;
-    const int spec_p = tp / P.nE, spec_q = tq / P.nE;
+    const int spec_p = P.cls_spec[tp], spec_q = P.cls_spec[tq];
     const float fs = (f0 < 0.0f || spec_p == spec_q) ? f0 : (float)P.cross_adh[spec_p] * f0;
     for (int d = 0; d < D; ++d) F[d] = fmaf(fs, dx[d], F[d]);
   }
@@ -1364,7 +1393,7 @@ __device__ inline void pair32_forces(const StepParams* __restrict__ Pp, const De
   const uint32_t ts = (uint32_t)step_ts(S);
   const int nE = P.nE;
   const int cshift = nE - 1;
-  const int spec_p = tp / nE;
+  const int spec_p = P.cls_spec[tp];
   const float ca_p = (float)P.cross_adh[spec_p];
   const int pidx = smeta[k] >> 3;
   const int cell_p = pidx >> cshift;
@@ -1392,8 +1421,8 @@ __device__ inline void pair32_forces(const StepParams* __restrict__ Pp, const De
     const int Rm = D == 3 ? P.reach_tt[tp][tq][1] : 0, Rr = P.reach_tt[tp][tq][D - 1];
     const Law32 Lw = law32(P, tp, tq);
     const float rca = (float)P.rca_tt[tp][tq], rcb = (float)P.rcb_tt[tp][tq];
-    const float cadh = (tq / nE == spec_p) ? 1.0f : ca_p;  // scale for f0 >= 0 (MD.cu:345-360)
-    const bool same_species_cells = nE == 2 && (tq / nE == spec_p);
+    const float cadh = (P.cls_spec[tq] == spec_p) ? 1.0f : ca_p;  // scale for f0 >= 0 (MD.cu:345-360)
+    const bool same_species_cells = nE == 2 && (P.cls_spec[tq] == spec_p);
     // This particle's largest cut-off against type tq (diameter bound of tq), with a margin
     // far above FP32 rounding: bins beyond it cannot hold a partner.  Columns are culled by
     // their x/y gap and each run is clipped to the bins its remaining radius reaches.
@@ -1568,7 +1597,7 @@ template <int D, int SH>
 __device__ inline void build_list_of(const StepParams& P, const Dev& S, int tp, int k, int sub, float4* win) {
   const float4* __restrict__ spos = (const float4*)S.spos;
   const int* __restrict__ start = S.start;
-  const int nE = P.nE, cshift = nE - 1, spec_p = tp / nE;
+  const int nE = P.nE, cshift = nE - 1, spec_p = P.cls_spec[tp];
   const int pidx = S.smeta[k] >> 3, cell_p = pidx >> cshift;
   if (SH == 0 || sub == 0) {
     for (int d = 0; d < D; ++d) S.xref[(size_t)d * S.P + pidx] = (float)S.pos[(size_t)d * S.P + pidx];
@@ -1597,7 +1626,7 @@ __device__ inline void build_list_of(const StepParams& P, const Dev& S, int tp, 
     if (Rx >= 0) {
       const int Ry = P.reach_tt[tp][tq][1], Rz = D == 3 ? P.reach_tt[tp][tq][2] : 0;
       const float rca = (float)P.rca_tt[tp][tq], rcb = (float)P.rcb_tt[tp][tq];
-      const bool same_species_cells = nE == 2 && (tq / nE == spec_p);
+      const bool same_species_cells = nE == 2 && (P.cls_spec[tq] == spec_p);
       const bool self_bucket = tq == tp;
       const float rcp = (fmaf(rca, me.w + (float)P.sigma_bound[tq], rcb) + skin) * 1.001f + 1e-6f;
       const float rcp2 = rcp * rcp;
@@ -1925,7 +1954,7 @@ __device__ inline void k_pair_list_body(const StepParams* __restrict__ Pp, const
   if (rebuild) build_list_of<D, SH>(P, S, tp, k, sub, bwin[threadIdx.x / WAVE]);
   const float4* __restrict__ spos = (const float4*)S.spos;
   const uint32_t ts = (uint32_t)step_ts(S);
-  const int nE = P.nE, spec_p = tp / nE;
+  const int spec_p = P.cls_spec[tp];
   const float ca_p = (float)P.cross_adh[spec_p];
   const int pidx = S.smeta[k] >> 3;
   const float4 me = spos[k];
@@ -1952,7 +1981,7 @@ __device__ inline void k_pair_list_body(const StepParams* __restrict__ Pp, const
       const int n = nlt[(size_t)tq * NL + L];
       if (n > 0) {
         const Law32 Lw = law32(P, tp, tq);
-        const float cadh = (tq / nE == spec_p) ? 1.0f : ca_p;  // scale for f0 >= 0 (MD.cu:345-360)
+        const float cadh = (P.cls_spec[tq] == spec_p) ? 1.0f : ca_p;  // scale for f0 >= 0 (MD.cu:345-360)
         if (RF) {
           il.rca = (float)P.rca_tt[tp][tq];
           il.rcb = (float)P.rcb_tt[tp][tq];

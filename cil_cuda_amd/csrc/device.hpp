@@ -166,7 +166,13 @@ struct LawEntry {
 
 struct StepParams {
   Box box;
+  // Element type t = species * nE + element.  The discs of a species whose law parameters are the same
+  // form one particle class: the sort, the stencils and the lists go by class, so such a two-disc
+  // species has half the buckets and half the runs per particle.  ntypes classes; every table indexed
+  // [type] below is by class.
   int nE, nspec, ntypes;
+  int cls[CIL_MAX_TYPES];       // element type -> class
+  int cls_spec[CIL_MAX_TYPES];  // class -> species
   int base[CIL_MAX_SPECIES];  // first cell slot of each species region
   int cap[CIL_MAX_SPECIES];
   LawEntry law[CIL_MAX_TYPES][CIL_MAX_TYPES];
@@ -199,6 +205,7 @@ struct StepParams {
   double rca_tt[CIL_MAX_TYPES][CIL_MAX_TYPES];    // force cut-off rc = rca*(s_p+s_q) + rcb
   double rcb_tt[CIL_MAX_TYPES][CIL_MAX_TYPES];
   double sigma_bound[CIL_MAX_TYPES];              // diameters the bins were sized for
+  double sigma_elem[CIL_MAX_TYPES];               // the same by element type
   int sort_range;   // buckets per workgroup of the one-launch sort (k_sort_multi); 0: general sort
   int pair_shift;   // stencil pair kernels: log2 of the lanes that share one particle
 };

@@ -11,7 +11,7 @@
 //                            (sorting network per lane, wave bitonic for large bins), so
 //                            every run is bit-reproducible
 //   spos        : float4 (bin-local x,y,z, sigma) in FP32 mode, double4 (global) in FP64
-//   smeta       : int32 [P]  particle*8 + element type
+//   smeta       : int32 [P]  particle*8 + class
 //   fpair/ppair : [D][P] / [P] pair forces and pressure partials, in sorted order
 #pragma once
 #include "device.hpp"
@@ -156,10 +156,9 @@ __device__ inline int bin_of(const StepParams& P, const double* x) {
   return b;
 }
 
-// Counting-sort key of particle p (slot index) at position x: element type major.
+// Counting-sort key of particle p (slot index) at position x: class major.
 __device__ inline int bucket_key(const StepParams& P, int p, int s, const double* x) {
-  int t = s * P.nE + (p % P.nE);
-  return t * P.nbins + bin_of(P, x);
+  return P.cls[s * P.nE + (p % P.nE)] * P.nbins + bin_of(P, x);
 }
 
 // ---------------------------------------------------------------------------------------

@@ -137,3 +137,67 @@ def test_two_level_list_lanes(gpu, cap):
 
 
 _SMALLEST = {}
+
+
+@pytest.mark.parametrize("mode", ["fp64", "fp32", "list32"])
+@pytest.mark.parametrize("law", [abi.LAW_SC, abi.LAW_HZ, abi.LAW_EA])
+@pytest.mark.parametrize("alike", [(1, 1), (1, 0), (0, 0)])
+def test_two_disc_classes(gpu, mode, law, alike):
+    """Two-disc species whose discs have the same law parameters (sorted as one class) or different ones
+    (two classes): forces and pair sets against the oracle."""
+    rng = np.random.default_rng(9 + law)
+    n, L = 120, 13.0
+    p = configs.base_params(2, 2, 2)
+    for s in range(2):
+        sp = p.species[s]
+        sp.spring, sp.k_harm = abi.SPRING_HARMONIC, 3.0
+        for e in range(2):
+            sp.sig_well[e] = 0.4 + 0.1 * s + (0.0 if alike[s] else 0.15 * e)
+            sp.eps_core[e] = 10.0 + (0.0 if alike[s] else 5.0 * e)
+            sp.eps_well[e] = 0.5 + 0.5 * s
+    p.species[1].cross_adhesion = 0.5
+    configs.set_law(p, law, 1.0)
+    p.precision = abi.PREC_FP64 if mode == "fp64" else abi.PREC_FP32
+    box = configs.make_box([L, L], [1, 1])
+    col = Colony(2, 2, [n, n], ncells=[n, n - 7])
+    for sp in col.species:
+        c = rng.uniform(0, L, (n, 2))
+        u = rng.normal(size=(n, 2))
+        u /= np.linalg.norm(u, axis=1, keepdims=True)
+        sp["pos"][:, 0], sp["pos"][:, 1] = c, np.mod(c + 0.6 * u, L)
+        sp["sigma"][:] = rng.uniform(0.8, 1.2, (n, 2))
+        sp["sigma"][:, 1] *= 1.2  # the diameter bounds differ by disc
+        sp["rest_len"][:] = 0.6
+        sp["state"][:] = abi.CS_CRAWLING
+    tol, floor = (1e-12, 0.0) if mode == "fp64" else (1e-5, 0.01)
+    worst, _, _ = _worst(p, box, col, tol, floor, skin=0.3 if mode == "list32" else 0.0)
+    assert worst <= 1.0, worst
+    q = abi.Params.from_buffer_copy(p)
+    q.precision = abi.PREC_FP64
+    orc = O.Oracle(q, box, traversal=1)
+    md = HipMD(p, box, [n, n])
+    md.upload(col)
+    assert np.array_equal(md.pairs(), orc.pairs(col))
+    md.close()
+    orc.close()
+
+
+def test_crowded_merged_bucket(gpu):
+    """More than 1,024 discs of a two-disc class in one bucket (each element type below that), in the
+    one-launch sort and, with a large capacity, in the general one."""
+    rng = np.random.default_rng(2)
+    n, L = 700, 2.0
+    for cap in (n, 40000):
+        p = configs.base_params(2, 1, 2)
+        p.species[0].spring, p.species[0].k_harm = abi.SPRING_HARMONIC, 1.0
+        for e in range(2):
+            p.species[0].sig_well[e], p.species[0].eps_core[e] = 0.5, 1.0
+        configs.set_law(p, abi.LAW_SC, 1.0)
+        box = configs.make_box([L, L], [1, 1])
+        col = Colony(2, 2, [cap], ncells=[n])
+        sp = col.species[0]
+        sp["pos"][:n] = rng.uniform(0, L, (n, 2, 2))
+        sp["sigma"][:n] = rng.uniform(0.9, 1.0, (n, 2))
+        sp["rest_len"][:n] = 0.6
+        worst, _, _ = _worst(p, box, col, 1e-12, 0.0)
+        assert worst <= 1.0, (cap, worst)
