@@ -1373,11 +1373,25 @@ __device__ __forceinline__ int run_coord(int sb) { return D == 3 ? (sb & 1023) :
 // Lanes, columns and runs as in k_pair64; a candidate's frame is its own bin's (FP32 local
 // coordinates), read from its packed bin beside its position, so a run crosses bins without a
 // look-up.  Lanes keep their own guard-band pairs (LDS) and resolve them before the sum.
-// At 131,071 particles (3D): 307 us with one thread per particle over single bins, 120 us with four.
-constexpr int PAIR32_UNROLL = 2;  // 4 need 98-112 VGPRs: 184 against 173 us per step
-template <int D>
-__device__ inline void pair32_forces(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
-  __shared__ int guard[256][GUARD_SLOTS];  // each lane's pairs inside the LJ guard band
+// Bound by instruction issue (131,071 particles in 3D: the vector units are busy 92 % of the time).
+// About one candidate in seven is in reach, so with 64 lanes the law would run for nearly every
+// candidate.  QUEUED (3D, up to eight lanes per particle): a lane queues its candidates in reach (LDS)
+// and the wave evaluates the queues together, in the order of the immediate form, so the sums have the
+// same bits.  With more lanes, or in 2D, a lane has few partners and the queue's extra loads cost more
+// than it saves.  131,071 particles: 307 us with one thread per particle over single bins, 120 us with
+// four lanes, 105 us queued (queues of 12; 8: the same, 16: 115, one workgroup less per CU).  Step,
+// immediate and queued: 4,001 particles 33 and 37 us (32 lanes), 30,011 66 and 66 (16), 64,011 102 and
+// 96 (8), 131,071 174 and 158 (4), 300,011 340 and 325, 1,000,003 830 and 752 (1); 32 two-disc 2D
+// colonies at once 87 and 95.
+constexpr int PAIR32_UNROLL = 4;  // candidates per pass, at most: 4 in 3D, 2 in 2D
+constexpr int PAIR32_QUEUE = 12;
+constexpr int PAIR32_QUEUE_SHIFT = 3;  // queued up to 2^3 lanes per particle
+template <int D, bool QUEUED>
+__device__ __forceinline__ void pair32_forces(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
+  __shared__ int guard[256][GUARD_SLOTS];        // each lane's pairs inside the LJ guard band
+  constexpr int U = QUEUED ? PAIR32_UNROLL : 2;
+  // each lane's candidates in reach, not yet evaluated: sorted slot, bin offsets
+  __shared__ uint2 queue[QUEUED ? PAIR32_QUEUE : 1][QUEUED ? 256 : 1];
   const StepParams& P = *Pp;
   const float4* __restrict__ spos = (const float4*)S.spos;
   const int* __restrict__ smeta = S.smeta;
@@ -1412,9 +1426,21 @@ __device__ inline void pair32_forces(const StepParams* __restrict__ Pp, const De
     one[d] = P.reach[d] == 0 && P.box.pbc[d];
   }
   const bool any_one = one[0] || one[1] || one[2];
-  const float wr = wid[D - 1], mr = xl[D - 1];
+  const float wr = wid[D - 1], iwr = (float)P.invw[D - 1], mr = xl[D - 1];
   float F[3] = {0.f, 0.f, 0.f}, pr = 0.f;
-  int nguard = 0;
+  int nguard = 0, nq = 0;
+  // the vector from p (at qx, qy, qr of the candidate's bin frame) to a candidate
+  auto delta = [&](const float4& r, float qx, float qy, float qr, float& dx, float& dy, float& dz) {
+    dx = r.x - qx;
+    dy = D == 3 ? r.y - qy : r.y - qr;
+    dz = D == 3 ? r.z - qr : 0.0f;
+    if (any_one) {
+      if (one[0]) dx -= (float)P.box.L[0] * rintf(dx * (float)P.box.invL[0]);
+      if (one[1]) dy -= (float)P.box.L[1] * rintf(dy * (float)P.box.invL[1]);
+      if (D == 3 && one[2]) dz -= (float)P.box.L[2] * rintf(dz * (float)P.box.invL[2]);
+    }
+    return fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+  };
   for (int tq = 0; tq < P.ntypes; ++tq) {
     const int Rx = P.reach_tt[tp][tq][0];
     if (Rx < 0) continue;
@@ -1428,9 +1454,33 @@ __device__ inline void pair32_forces(const StepParams* __restrict__ Pp, const De
     // their x/y gap and each run is clipped to the bins its remaining radius reaches.
     const float rcp = fmaf(rca, me.w + (float)P.sigma_bound[tq], rcb) * 1.001f + 1e-6f;
     const float rcp2 = rcp * rcp;
+    const float rct = rca * 1.0001f, rcu = fmaf(rca, me.w, rcb) * 1.0001f;  // a candidate's cut-off, widened
+    // evaluates the lane's queued candidates, in their order
+    auto flush = [&]() {
+      for (int h = 0; h < nq; ++h) {
+        const uint2 e = queue[h][threadIdx.x];
+        const int j = (int)e.x;
+        if (j == k) continue;
+        const float4 r = spos[j];
+        if (same_species_cells && ((smeta[j] >> 3) >> cshift) == cell_p) continue;
+        const float qx = me.x - (float)((int)(e.y << 24) >> 24) * wid[0];
+        const float qy = me.y - (float)((int)(e.y << 16) >> 24) * wid[1];
+        float dx, dy, dz, f0, temp;
+        const float r2 = delta(r, qx, qy, mr - (float)((int)e.y >> 16) * wr, dx, dy, dz);
+        bool contact;
+        if (!pair_term32<D>(P, S, Lw, guard[threadIdx.x], j, pidx, me.w, r.w, r2, ts, dx, dy, nguard, f0, contact, temp)) continue;
+        const float fs = f0 < 0.0f ? f0 : cadh * f0;
+        F[0] = fmaf(fs, dx, F[0]);
+        F[1] = fmaf(fs, dy, F[1]);
+        if (D == 3) F[2] = fmaf(fs, dz, F[2]);
+        if (contact && temp != 0.0f) pr -= fs / temp;
+      }
+      nq = 0;
+    };
     const int side = 2 * Rm + 1, ncol = (2 * Rx + 1) * side;
+    const float iside = rcp32((float)side);
     for (int c = sub; c < ncol; c += lanes) {
-      const int cx = D == 3 ? c / side : c;
+      const int cx = D == 3 ? (int)(((float)c + 0.5f) * iside) : c;  // c / side (both far below 2^20)
       const int ox = cx - Rx, oy = D == 3 ? c - cx * side - Rm : 0;
       int nx = bc[0] + ox;
       if (P.box.pbc[0]) nx = nx < 0 ? nx + P.ns[0] : (nx >= P.ns[0] ? nx - P.ns[0] : nx);
@@ -1451,8 +1501,9 @@ __device__ inline void pair32_forces(const StepParams* __restrict__ Pp, const De
       if (rem < 0.0f) continue;
       int lo = -Rr, hi = Rr;
       if (!one[D - 1]) {
-        const float sr = sqrtf(rem);
-        const int a = (int)floorf((loc[D - 1] + sr) / wr), b = (int)ceilf((loc[D - 1] - sr) / wr) - 1;
+        // the radius margin (1e-3 of the cut-off) covers the rounding of the root and the reciprocal
+        const float sr = sqrt32(rem);
+        const int a = (int)floorf((loc[D - 1] + sr) * iwr), b = (int)ceilf((loc[D - 1] - sr) * iwr) - 1;
         hi = a < Rr ? a : Rr;
         lo = b > -Rr ? b : -Rr;
         if (lo > hi) continue;
@@ -1460,45 +1511,70 @@ __device__ inline void pair32_forces(const StepParams* __restrict__ Pp, const De
       int z0[2], z1[2], zo[2];
       const int nseg = run_segments(P, D - 1, bc[D - 1], lo, hi, z0, z1, zo);
       const int base = tq * P.nbins + row * P.ns[D - 1];
+      const unsigned col = (unsigned)(ox & 255) | (unsigned)(oy & 255) << 8;
       for (int sg = 0; sg < nseg; ++sg) {
         const int unwrap = zo[sg] - z0[sg];  // bin coordinate along the run -> offset from p's bin
         const int j1 = start[base + z1[sg] + 1];
-        for (int j = start[base + z0[sg]]; j < j1; j += PAIR32_UNROLL) {
-          float4 r[PAIR32_UNROLL];
-          int sb[PAIR32_UNROLL];
+        for (int j = start[base + z0[sg]]; j < j1; j += U) {
+          float4 r[U];
+          int sb[U];
+          if constexpr (QUEUED) {
+            // byte offsets in 32 bits (a sorted slot is below 2^28); the arrays hold PAIR32_UNROLL
+            // records more than there are slots
+            const float4* rj = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(spos) + ((unsigned)j << 4));
+            const int* bj = reinterpret_cast<const int*>(reinterpret_cast<const char*>(sbin) + ((unsigned)j << 2));
 #pragma unroll
-          for (int q = 0; q < PAIR32_UNROLL; ++q) {
-            const int jj = j + q < j1 ? j + q : j1 - 1;
-            r[q] = spos[jj];
-            sb[q] = sbin[jj];
-          }
-#pragma unroll
-          for (int q = 0; q < PAIR32_UNROLL; ++q) {
-            const float qr = mr - (float)(run_coord<D>(sb[q]) + unwrap) * wr;
-            float dx = r[q].x - qx, dy = D == 3 ? r[q].y - qy : r[q].y - qr, dz = D == 3 ? r[q].z - qr : 0.0f;
-            if (any_one) {
-              if (one[0]) dx -= (float)P.box.L[0] * rintf(dx * (float)P.box.invL[0]);
-              if (one[1]) dy -= (float)P.box.L[1] * rintf(dy * (float)P.box.invL[1]);
-              if (D == 3 && one[2]) dz -= (float)P.box.L[2] * rintf(dz * (float)P.box.invL[2]);
+            for (int q = 0; q < U; ++q) {
+              r[q] = rj[q];
+              sb[q] = bj[q];
             }
-            const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-            const float ssum = r[q].w + me.w;
-            const float rc = fmaf(rca, ssum, rcb);
-            const int jq = j + q;
-            if (jq >= j1 || r2 > rc * rc * 1.0001f || jq == k) continue;
-            if (same_species_cells && ((smeta[jq] >> 3) >> cshift) == cell_p) continue;
-            float f0, temp;
-            bool contact;
-            if (!pair_term32<D>(P, S, Lw, guard[threadIdx.x], jq, pidx, me.w, r[q].w, r2, ts, dx, dy, nguard, f0, contact, temp)) continue;
-            const float fs = f0 < 0.0f ? f0 : cadh * f0;
-            F[0] = fmaf(fs, dx, F[0]);
-            F[1] = fmaf(fs, dy, F[1]);
-            if (D == 3) F[2] = fmaf(fs, dz, F[2]);
-            if (contact && temp != 0.0f) pr -= fs / temp;
+#pragma unroll
+            for (int q = 0; q < U; ++q) {
+              const int orun = run_coord<D>(sb[q]) + unwrap;
+              float dx, dy, dz;
+              const float r2 = delta(r[q], qx, qy, mr - (float)orun * wr, dx, dy, dz);
+              const float rc = fmaf(rct, r[q].w, rcu);
+              if (j + q >= j1 || r2 > rc * rc) continue;
+              queue[nq][threadIdx.x] = make_uint2((unsigned)(j + q), col | (unsigned)orun << 16);
+              ++nq;
+            }
+            if (__any(nq > PAIR32_QUEUE - U)) flush();
+          } else {
+#pragma unroll
+            for (int q = 0; q < U; ++q) {
+              const int jj = j + q < j1 ? j + q : j1 - 1;
+              r[q] = spos[jj];
+              sb[q] = sbin[jj];
+            }
+#pragma unroll
+            for (int q = 0; q < U; ++q) {
+              const float qr = mr - (float)(run_coord<D>(sb[q]) + unwrap) * wr;
+              float dx = r[q].x - qx, dy = D == 3 ? r[q].y - qy : r[q].y - qr, dz = D == 3 ? r[q].z - qr : 0.0f;
+              if (any_one) {
+                if (one[0]) dx -= (float)P.box.L[0] * rintf(dx * (float)P.box.invL[0]);
+                if (one[1]) dy -= (float)P.box.L[1] * rintf(dy * (float)P.box.invL[1]);
+                if (D == 3 && one[2]) dz -= (float)P.box.L[2] * rintf(dz * (float)P.box.invL[2]);
+              }
+              const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+              const float ssum = r[q].w + me.w;
+              const float rc = fmaf(rca, ssum, rcb);
+              const int jq = j + q;
+              if (jq >= j1 || r2 > rc * rc * 1.0001f || jq == k) continue;
+              if (same_species_cells && ((smeta[jq] >> 3) >> cshift) == cell_p) continue;
+              float f0, temp;
+              bool contact;
+              if (!pair_term32<D>(P, S, Lw, guard[threadIdx.x], jq, pidx, me.w, r[q].w, r2, ts, dx, dy, nguard, f0, contact, temp)) continue;
+              const float fs = f0 < 0.0f ? f0 : cadh * f0;
+              F[0] = fmaf(fs, dx, F[0]);
+              F[1] = fmaf(fs, dy, F[1]);
+              if (D == 3) F[2] = fmaf(fs, dz, F[2]);
+              if (contact && temp != 0.0f) pr -= fs / temp;
+            }
           }
         }
       }
     }
+    if (QUEUED) flush();
   }
   if (nguard > 0) {
     float g[3] = {0.f, 0.f, 0.f};
@@ -1517,15 +1593,15 @@ __device__ inline void pair32_forces(const StepParams* __restrict__ Pp, const De
   }
   if (group_sum(nguard, lanes) > GUARD_SLOTS) atomicOr(S.err, (unsigned)ERR_GUARD);
 }
-template <int D>
+template <int D, bool QUEUED>
 __device__ inline void k_pair32_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
-  pair32_forces<D>(Pp, S, bid);
+  pair32_forces<D, QUEUED>(Pp, S, bid);
   clear_counts(*Pp, S, bid * (int)blockDim.x + (int)threadIdx.x, S.P << Pp->pair_shift);
 }
 #define PAIR32_WPE 5  // six waves per SIMD spill
-template <int D>
+template <int D, bool QUEUED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PAIR32_WPE)))
-k_pair32(const StepParams* __restrict__ Pp, Dev S) { k_pair32_body<D>(Pp, S, xcd_block_chunked(blockIdx.x, gridDim.x)); }
+k_pair32(const StepParams* __restrict__ Pp, Dev S) { k_pair32_body<D, QUEUED>(Pp, S, xcd_block_chunked(blockIdx.x, gridDim.x)); }
 
 // ======================================================================================
 // Neighbour-list mode (FP32).  A list entry is (sorted index << 10) | bin offset code; the

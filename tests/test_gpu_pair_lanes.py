@@ -201,3 +201,15 @@ def test_crowded_merged_bucket(gpu):
         sp["rest_len"][:n] = 0.6
         worst, _, _ = _worst(p, box, col, 1e-12, 0.0)
         assert worst <= 1.0, (cap, worst)
+
+
+@pytest.mark.parametrize("law", [abi.LAW_SC, abi.LAW_HZ])
+@pytest.mark.parametrize("capacity", [65536, 65537, 200000, 600000])
+@pytest.mark.parametrize("periodic", [0, 1])
+def test_crowded_queues(gpu, law, capacity, periodic):
+    """Far more partners in reach per lane than a lane's queue holds (FP32, 3D, eight lanes to one)."""
+    p, box, col = _colony(3, 900, 6.0, periodic, law, capacity, 21, stray=0 if periodic else 9)
+    p.precision = abi.PREC_FP32
+    p.max_disp = 0.0
+    worst, pr, ref = _worst(p, box, col, 1e-5, 0.01 if periodic else 0.02)
+    assert worst <= 1.0, worst
