@@ -2,19 +2,20 @@
 // the C ABI of include/cil_hip.h.
 //
 // Step (one Euler(ts) of CIL.cu:1013-1020), kernels in launch order:
-//   k_update     per cell: lazy intra-cell force (CIL.cu:30-100) + sorted pair force ->
-//                fused overdamped update (CIL.cu:902-939); when no division is configured
-//                it also emits the particle's bin key and arrival rank (counting sort pass 1)
-//   [division]   k_div_* flag / prefix-sum / append in parent order (CIL.cu:469-619)
-//   [k_keys]     bin key + rank, when division moved particles
-//   [k_noise]    Wiener deviates per cell (CIL.cu:793-818), reference noise mode only
-//   k_scan_*     exclusive prefix sum of bin counts
-//   k_scatter    particle -> slot in bin order
-//   k_binsort    one wavefront per bucket (element type x spatial bin): bitonic sort of the
-//                bucket's particle ids (deterministic order), gather of bin-local coordinates
-//   k_pair<T>    one thread per sorted particle: full-shell gather over the per-type-pair
-//                stencil, walked as contiguous z-runs; canonical (lower-UID) orientation per
-//                pair so asymmetric terms match the reference
+//   k_update     per cell: noise, lazy intra-cell force (CIL.cu:30-100) + sorted pair force ->
+//                fused overdamped update (CIL.cu:902-939); it also emits the particle's bucket
+//                and counts it (counting sort pass 1)
+//   [division]   flags, prefix sum, append in parent order (CIL.cu:469-619): one launch
+//                (k_div_fused) below 2^15 cells, k_div_* above
+//   [k_noise]    Wiener deviates per cell (CIL.cu:793-818) kept between calls; a run's own steps
+//                draw them in k_update
+//   k_sort_multi the rest of the counting sort in one launch, up to 2^16 particle slots; above,
+//                k_scan_* (exclusive prefix sum of the counts), k_scatter (particle -> slot) and
+//                k_binsort (each bucket's particles in index order, bin-local coordinates).
+//                A bucket is (particle class, spatial bin)
+//   k_pair64, k_pair32   several lanes per sorted particle: full-shell gather over the per-class-pair
+//                stencil, walked as contiguous runs; canonical (lower-UID) orientation per
+//                pair so asymmetric terms match the reference.  k_pair: the generic FP32 form
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -651,8 +652,8 @@ __global__ void __launch_bounds__(256) k_sort_all(const StepParams* __restrict__
 }
 
 // ======================================================================================
-// Pair forces.  Thread per sorted particle: a wavefront holds 64 consecutive particles of
-// one element type, i.e. a short run of bins along z.  For each source type the stencil
+// Pair forces.  One or more lanes per sorted particle: a wavefront holds consecutive particles of
+// one class, i.e. a short run of bins along z.  For each source type the stencil
 // (reach per type pair) is walked as (x, y) columns; the z-run of a column is one contiguous
 // range of the sorted array, walked in a single loop that only tracks bin boundaries for
 // the periodic shift.  Law parameters of the (target, source) type pair sit in registers;
@@ -844,7 +845,7 @@ __device__ inline void pair32(const StepParams& P, const Dev& S, const PairLaw& 
   if (contact && P.pressure && temp != 0.0f) *pr -= fs / temp;
 }
 
-// Bucket of (element type t, spatial bin coordinates).
+// Bucket of (class t, spatial bin coordinates).
 __device__ inline int bucket_of(const StepParams& P, int t, int x, int y, int z) {
   int b = P.box.dim == 3 ? (x * P.ns[1] + y) * P.ns[2] + z : x * P.ns[1] + y;
   return t * P.nbins + b;
@@ -928,7 +929,7 @@ __device__ inline int z_segments(const StepParams& P, int bz, int R, int* z0, in
   return 1;
 }
 
-// Wave w of the per-type layout: the sorted array is type-major; each element type's range is
+// Wave w of the per-type layout: the sorted array is type-major; each class's range is
 // cut into chunks of `per` particles, one per wave, so the type is wave-uniform.  False beyond
 // the last chunk.
 __device__ inline bool wave_type_chunk(const StepParams& P, const int* __restrict__ start, int w, int per, int* tp_out,
@@ -1209,7 +1210,7 @@ __device__ inline void k_pair_body(const StepParams* __restrict__ Pp, const Dev&
 __global__ void __launch_bounds__(256) k_pair(const StepParams* __restrict__ Pp, Dev S) { k_pair_body(Pp, S, xcd_block_chunked(blockIdx.x, gridDim.x)); }
 
 // Lean FP32 pair kernel (k_pair32, fast mode), specialised on the dimension.  Waves are laid out
-// per element type (the sorted array is type-major), so the target type, its species, the law of
+// per class (the sorted array is type-major), so the target type, its species, the law of
 // each (target, source) type pair, the stencil reach and the cross-adhesion choice are wave-uniform
 // (scalar registers).  Single-disc cells: the same-cell exclusion is j == k, so the inner loop
 // reads only each candidate's sorted record and packed bin.
@@ -1610,9 +1611,9 @@ k_pair32(const StepParams* __restrict__ Pp, Dev S) { k_pair32_body<D, QUEUED>(Pp
 // ======================================================================================
 __device__ inline int list_code(int ox, int oy, int oz) { return ((ox + 4) * 9 + (oy + 4)) * 9 + (oz + 4); }
 
-// Wave -> (element type, sorted index) of the list kernels.  Workgroups are dispatched to the
+// Wave -> (class, sorted index) of the list kernels.  Workgroups are dispatched to the
 // XCDs round-robin (workgroup b runs on XCD b % 8), so XCD x takes the x-th contiguous eighth
-// of every element type's waves: each XCD walks one compact region of space, whose neighbour
+// of every class's waves: each XCD walks one compact region of space, whose neighbour
 // positions stay in its own L2, and gets an equal share of each type (types differ in list
 // length).  Within an XCD the waves run type by type.  The grid holds at least
 // ceil((sum over types of ceil(waves_t / 8)) / waves per block) workgroups per XCD; waves
@@ -1656,7 +1657,7 @@ __device__ __forceinline__ int wave_max_all(int v) {
 // Candidate window of the list build: sorted positions staged per wave in LDS.
 constexpr int BUILD_WIN = 160;
 
-// List build of sorted particle k (element type tp), run by the list pair kernel when this
+// List build of sorted particle k (class tp), run by the list pair kernel when this
 // pass rebuilds: every pair within its own cut-off plus the skin, found with the culled
 // stencil walk of k_pair32; records the build positions.  Only k's own list is written, so
 // the pair loop of the same lane can read it right after.  Entries are stored in groups of

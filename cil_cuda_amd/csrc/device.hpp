@@ -194,7 +194,7 @@ struct StepParams {
   cil_wall walls[CIL_MAX_WALLS];
   cil_species sp[CIL_MAX_SPECIES];
   // bins: spatial grid ns[0] x ns[1] x ns[2]; particles are counting-sorted into buckets
-  // (element type, spatial bin), bucket = type * nbins + bin
+  // (class, spatial bin), bucket = type * nbins + bin
   int ns[3];
   double w[3];      // bin widths (L/ns)
   double invw[3];
