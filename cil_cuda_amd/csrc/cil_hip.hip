@@ -2289,7 +2289,8 @@ __device__ inline void list_track(const StepParams& P, const Dev& S, size_t p, c
 }
 
 // flags: forces are the materialised ones; a step inside a chunk of launched steps, whose velocities the
-// next step replaces unread (they are stored only where the intra force reads them).
+// next step replaces unread (they are stored only where the intra force reads them; never set in replays
+// of the sequential stream, whose walk reads all of them).
 constexpr int UPD_MATERIALIZED = 1, UPD_MID_CHUNK = 4;
 constexpr int UPD_STORED_NOISE = 2;  // host only: the kernel that reads the pass's noise from the arrays
 template <typename T, int DIM, int NE, bool DRAW>

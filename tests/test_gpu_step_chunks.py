@@ -54,6 +54,33 @@ def test_chunked_steps_match_single_steps(gpu, build):
         assert np.array_equal(a.flat(f), b.flat(f)), f
 
 
+def test_replayed_stream_reads_every_velocity(gpu):
+    """The reference's sequential stream (dSFMT): a single disc at rest draws a direction at every force
+    pass, whatever its motility, so each step's velocity must be there for the next pass.  Discs too far
+    apart to touch, no motility, dividing: chunked, single and the oracle's steps make the same draws."""
+    p, box, col = configs.theta_2d_hz(n_cells=12, L=60.0, seed=6)
+    p.species[0].motility[0] = 0.0
+    p.rng = abi.RNG_DSFMT
+    col.species[0]["pos"][:12, 0] = 8.0 + 15.0 * np.stack([np.arange(12) % 4, np.arange(12) // 4], 1)
+    col.species[0]["vel"][:12, 0, 0] = 0.3
+    a = _run(p, box, col, [(70, 0), (5, 0)])
+    b = _run(p, box, col, [(1, 0)] * 75)
+    ref = col.copy()
+    orc = O.Oracle(p, box, traversal=1)
+    orc.set_rng(O.RNG_DSFMT, p.seed)
+    orc.forces(ref, 0)
+    orc.step(ref, 75, 0)
+    assert a.ncells() == b.ncells() == ref.ncells() and a.ncells()[0] > 12
+    for f in ("pos", "vel", "frc", "sigma", "pressure", "theta", "ang_vel", "tswitch", "t0"):
+        assert np.array_equal(a.flat(f), b.flat(f)), f
+    assert np.array_equal(a.flat("t0"), ref.flat("t0"))
+    # the spans come from the stream's normal draws: one draw more or less changes them altogether
+    assert np.allclose(a.flat("ang_vel"), ref.flat("ang_vel"), rtol=1e-11)
+    d = a.flat("pos") - ref.flat("pos")
+    d -= box.length[0] * np.round(d / box.length[0])
+    assert np.max(np.abs(d)) <= 1e-9
+
+
 @pytest.mark.parametrize("active", [0, 1])
 def test_noise_of_held_forces_keeps_its_step_index(gpu, active):
     """Forces held from index 0, then steps from index 40: the first step uses the noise drawn at 0."""
