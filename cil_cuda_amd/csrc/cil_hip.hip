@@ -252,15 +252,17 @@ __device__ inline void unpack_bin(const StepParams& P, int s, int* bc) {
   }
 }
 
+// Sorted record of particle p: FP32 coordinates local to its bin, FP64 ones in the box (where a dimension
+// is periodic), so that a stencil column's image shift alone gives the minimum image.
 template <typename T>
 __device__ inline void write_sorted(const StepParams& P, const Dev& S, const int* bc, int k, int p);
 
 template <>
 __device__ inline void write_sorted<float>(const StepParams& P, const Dev& S, const int* bc, int k, int p) {
   float4 r;
-  r.x = (float)(S.pos[p] - bc[0] * P.w[0]);
-  r.y = (float)(S.pos[(size_t)S.P + p] - bc[1] * P.w[1]);
-  r.z = P.box.dim == 3 ? (float)(S.pos[2 * (size_t)S.P + p] - bc[2] * P.w[2]) : 0.0f;
+  r.x = (float)(box_image(P.box, 0, S.pos[p]) - bc[0] * P.w[0]);
+  r.y = (float)(box_image(P.box, 1, S.pos[(size_t)S.P + p]) - bc[1] * P.w[1]);
+  r.z = P.box.dim == 3 ? (float)(box_image(P.box, 2, S.pos[2 * (size_t)S.P + p]) - bc[2] * P.w[2]) : 0.0f;
   r.w = (float)S.sigma[p];
   ((float4*)S.spos)[k] = r;
 }
@@ -268,9 +270,9 @@ template <>
 __device__ inline void write_sorted<double>(const StepParams& P, const Dev& S, const int* bc, int k, int p) {
   (void)bc;
   double4 r;
-  r.x = S.pos[p];
-  r.y = S.pos[(size_t)S.P + p];
-  r.z = P.box.dim == 3 ? S.pos[2 * (size_t)S.P + p] : 0.0;
+  r.x = box_image(P.box, 0, S.pos[p]);
+  r.y = box_image(P.box, 1, S.pos[(size_t)S.P + p]);
+  r.z = P.box.dim == 3 ? box_image(P.box, 2, S.pos[2 * (size_t)S.P + p]) : 0.0;
   r.w = S.sigma[p];
   ((double4*)S.spos)[k] = r;
 }

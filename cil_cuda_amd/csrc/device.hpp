@@ -124,6 +124,12 @@ __device__ inline double box_dist(const Box& b, double* r12, const double* r1, c
   return ans;
 }
 
+// Image of coordinate x inside the box along a periodic dimension; x itself along an open one.  Updates
+// keep discs in the box, but an uploaded position may lie any number of box lengths outside.
+__device__ inline double box_image(const Box& b, int d, double x) {
+  return !b.pbc[d] || (x >= 0.0 && x < b.L[d]) ? x : x - floor(x / b.L[d]) * b.L[d];
+}
+
 // BoundingBox::updatePos(r, v, dt) (Utils.hpp:561-566)
 __device__ inline double box_update1(const Box& b, int d, double r, double v, double dt) {
   return b.pbc[d] ? wrap_fmod(r + dt * v + b.L[d], b.L[d]) : r + v * dt;

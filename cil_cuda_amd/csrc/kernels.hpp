@@ -143,8 +143,10 @@ __device__ inline bool cell_active(const StepParams& P, const int* ncells, int c
   return c < ncells[s];
 }
 
+// Bin along dimension d of coordinate x: of its image in the box where the dimension is periodic
+// (box_image), the edge bin outside an open box.
 __device__ inline int bin_coord(const StepParams& P, int d, double x) {
-  int b = (int)floor(x * P.invw[d]);
+  int b = (int)floor(box_image(P.box, d, x) * P.invw[d]);
   b = b < 0 ? 0 : b;
   b = b > P.ns[d] - 1 ? P.ns[d] - 1 : b;
   return b;

@@ -237,7 +237,8 @@ typedef struct cil_ctx cil_ctx;
 int cil_hip_create(const cil_params* params, const cil_box* box, const int* capacity, cil_ctx** out);
 int cil_hip_destroy(cil_ctx* ctx);
 
-/* Copy the host colony to the device (all species). */
+/* Copy the host colony to the device (all species).  A position outside a periodic box stands for its
+ * image inside, any number of box lengths away. */
 int cil_hip_upload(cil_ctx* ctx, const cil_species_view* views, int nspec);
 
 /* Run the Euler phase order (CIL.cu:1013-1020) `nsteps` times; *ts is incremented per step
