@@ -73,6 +73,10 @@ __device__ inline int xcd_block_chunked(int b, int nblk) {
 // ======================================================================================
 // Bin keys
 // ======================================================================================
+// RANK: the particle's arrival rank in its bucket is kept (slot), so that the scatter places it without an
+// atomic of its own.  For the persistent sort, whose keys are a phase between grid barriers; the update's
+// and k_keys' counting adds want no answer.
+template <bool RANK>
 __device__ inline void k_keys_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
   const StepParams& P = *Pp;
   if (sort_skipped(S)) return;
@@ -96,9 +100,10 @@ __device__ inline void k_keys_body(const StepParams* __restrict__ Pp, const Dev&
   }
   int b = bucket_key(P, p, s, x);
   S.key[p] = b;
-  atomicAdd(&S.count[b], 1);
+  if (RANK) S.slot[p] = atomicAdd(&S.count[b], 1);
+  else atomicAdd(&S.count[b], 1);
 }
-__global__ void k_keys(const StepParams* __restrict__ Pp, Dev S) { k_keys_body(Pp, S, (int)blockIdx.x); }
+__global__ void k_keys(const StepParams* __restrict__ Pp, Dev S) { k_keys_body<false>(Pp, S, (int)blockIdx.x); }
 
 // ======================================================================================
 // Exclusive prefix sum (2 small kernels): 4096 items per block of 256 threads.
@@ -198,15 +203,17 @@ __global__ void __launch_bounds__(256) k_scan_add(int* __restrict__ out, const i
 // ======================================================================================
 // Scatter and per-bin sort + gather
 // ======================================================================================
+template <bool RANK>
 __device__ inline void k_scatter_body(const Dev& S, int bid) {
   if (sort_skipped(S)) return;
   int p = bid * blockDim.x + threadIdx.x;
   if (p >= S.P) return;
   int b = S.key[p];
   if (b < 0) return;
-  S.idx[atomicAdd(&S.count[b], 1)] = p;  // the scan left the bucket's start in its count
+  if (RANK) S.idx[S.start[b] + S.slot[p]] = p;
+  else S.idx[atomicAdd(&S.count[b], 1)] = p;  // the scan left the bucket's start in its count
 }
-__global__ void k_scatter(Dev S) { k_scatter_body(S, (int)blockIdx.x); }
+__global__ void k_scatter(Dev S) { k_scatter_body<false>(S, (int)blockIdx.x); }
 
 // Orders this wave's LDS accesses across lanes (wave-scope fence + wave barrier).
 __device__ inline void wave_lds_sync() {
@@ -634,7 +641,7 @@ __global__ void __launch_bounds__(256) k_sort_all(const StepParams* __restrict__
   const StepParams& P = *Pp;
   const unsigned G = gridDim.x;
   const int np = (S.P + 255) / 256;
-  for (int vb = blockIdx.x; vb < np; vb += (int)G) k_keys_body(Pp, S, vb);
+  for (int vb = blockIdx.x; vb < np; vb += (int)G) k_keys_body<true>(Pp, S, vb);
   bool ok = grid_barrier(sync, 1, S.err);
   const int nt = P.nbuckets > 0 ? (P.nbuckets + SCAN_TILE - 1) / SCAN_TILE : 1;
   if (ok)
@@ -643,10 +650,10 @@ __global__ void __launch_bounds__(256) k_sort_all(const StepParams* __restrict__
   const int na = P.nbuckets > 0 ? (P.nbuckets + 255) / 256 : 1;
   if (ok)
     for (int vb = blockIdx.x; vb < na; vb += (int)G)
-      k_scan_add_body(S.start, S.blocksum, P.nbuckets, S.start + P.nbuckets, S.count, vb);
+      k_scan_add_body(S.start, S.blocksum, P.nbuckets, S.start + P.nbuckets, nullptr, vb);
   ok = ok && grid_barrier(sync, 3, S.err);
   if (ok)
-    for (int vb = blockIdx.x; vb < np; vb += (int)G) k_scatter_body(S, vb);
+    for (int vb = blockIdx.x; vb < np; vb += (int)G) k_scatter_body<true>(S, vb);
   ok = ok && grid_barrier(sync, 4, S.err);
   if (ok) k_binsort_body<T>(Pp, S, (int)blockIdx.x, (int)G);
   __syncthreads();
@@ -1929,9 +1936,14 @@ struct InnerList {
   }
 };
 
-template <int D, int LC, bool MI, bool SH, bool RF>
+// Guard-band slots of a list: by its number (one lane per particle: the number is at hand and a pointer held
+// over the loop spills) or by its pointer.
+__device__ __forceinline__ int* guard_slots(const Dev& S, unsigned list) { return S.gslot + (size_t)list * GUARD_SLOTS; }
+__device__ __forceinline__ int* guard_slots(const Dev&, int* slots) { return slots; }
+
+template <int D, int LC, bool MI, bool SH, bool RF, typename Guard>
 __device__ __forceinline__ void list_segment(const StepParams& P, const Dev& S, const Law32& Lw, const float4* tab,
-                                             const float4& me, int* gslot, int pidx, uint32_t ts, float cadh, int n,
+                                             const float4& me, Guard gslot, int pidx, uint32_t ts, float cadh, int n,
                                              const char* __restrict__ nlb, unsigned& off, unsigned stride, float& Fx,
                                              float& Fy, float& Fz, float& pr, int& nguard, InnerList& il) {
   const float4* __restrict__ spos = (const float4*)S.spos;
@@ -1954,7 +1966,7 @@ __device__ __forceinline__ void list_segment(const StepParams& P, const Dev& S, 
       bool guard;
       f0 = lj_term32<SH>(Lw, r.w + me.w, r2, &guard);
       if (guard) {  // rare: recorded for the exact FP64 decision after the loop
-        if (nguard < GUARD_SLOTS) gslot[nguard] = (int)(e >> 10);
+        if (nguard < GUARD_SLOTS) guard_slots(S, gslot)[nguard] = (int)(e >> 10);
         ++nguard;
       }
     } else if (LC == CIL_LAW_SC) {
@@ -2042,7 +2054,10 @@ __device__ inline void k_pair_list_body(const StepParams* __restrict__ Pp, const
   const size_t NP = (size_t)S.P, NL = NP << SH, L = ((size_t)k << SH) + sub;  // lanes' lists, this lane's
   const unsigned stride = 16u * (unsigned)NL;
   unsigned off = 16u * (unsigned)L;
-  int* const gslot = S.gslot + L * GUARD_SLOTS;
+  const auto gslot = [&] {
+    if constexpr (SH == 0) return (unsigned)L;
+    else return S.gslot + L * GUARD_SLOTS;
+  }();
   float Fx = 0.f, Fy = 0.f, Fz = 0.f, pr = 0.f;
   int nguard = 0;
   // two-level lists: a refresh pass evaluates the outer list and writes the inner one; other
@@ -2100,7 +2115,7 @@ __device__ inline void k_pair_list_body(const StepParams* __restrict__ Pp, const
   else run_types(std::false_type{});
   if (nguard > 0) {
     float g[3] = {0.f, 0.f, 0.f};
-    guard_force(P, S, k, gslot, nguard, g);
+    guard_force(P, S, k, guard_slots(S, gslot), nguard, g);
     Fx += g[0];
     Fy += g[1];
     if (D == 3) Fz += g[2];

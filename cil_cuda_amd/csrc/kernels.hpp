@@ -45,7 +45,7 @@ struct Dev {
   int* count;
   int* start;       // [nbins+1]
   int* blocksum;
-  int* slot;        // [P] k_sort_multi: a bucket's particles in arrival order
+  int* slot;        // [P] k_sort_multi: a bucket's particles in arrival order; k_sort_all: arrival ranks
   int* idx;
   int* inv;
   void* spos;
