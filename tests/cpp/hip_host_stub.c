@@ -1,10 +1,11 @@
 /* A HIP runtime of two devices without any: "device" memory is host memory, kernels do nothing.  It counts
- * what is allocated while each device is current. */
+ * what is allocated while each device is current, and the launches. */
 #include <stdlib.h>
 #include <string.h>
 
-static int current, allocs[2];
+static int current, allocs[2], launches;
 int stub_allocs(int dev) { return allocs[dev]; }
+int stub_launches(void) { return launches; }
 
 #define NOTE allocs[current]++
 int hipGetDeviceCount(int* n) { *n = 2; return 0; }
@@ -44,7 +45,7 @@ int hipGraphInstantiate(void** e, void* g, void* n, char* b, size_t k) {
   (void)g; (void)n; (void)b; (void)k; *e = 0; return 0;
 }
 int hipGraphLaunch(void* e, void* s) { (void)e; (void)s; return 0; }
-int hipLaunchKernel(const void* f, ...) { (void)f; return 0; }
+int hipLaunchKernel(const void* f, ...) { (void)f; launches++; return 0; }
 int __hipPushCallConfiguration(void) { return 0; }
 int __hipPopCallConfiguration(void* g, void* b, size_t* shm, void** st) {
   memset(g, 0, 12); memset(b, 0, 12); *shm = 0; *st = 0; return 0;
