@@ -1402,12 +1402,26 @@ __device__ __forceinline__ int run_coord(int sb) { return D == 3 ? (sb & 1023) :
 constexpr int PAIR32_UNROLL = 4;  // candidates per pass, at most: 4 in 3D, 2 in 2D
 constexpr int PAIR32_QUEUE = 12;
 constexpr int PAIR32_QUEUE_SHIFT = 3;  // queued up to 2^3 lanes per particle
-template <int D, bool QUEUED>
+// SPLIT (batches of small 3D colonies, choose_lane_split): a lane takes the shares of four of the 32 lanes that
+// such a colony gives a particle, in turn, and adds their sums in the order of the lanes' tree, so that the
+// forces have the bits of the colony alone.  Alone, a colony of 5,000 needs the 32 lanes to fill the chip
+// (46 us a step against 260 with one); a batch fills it anyway, and lanes on different columns of one
+// particle wait for the longest column.  Step, 32 lanes at once and 8 in four turns: 64 colonies of 5,000 608
+// and 478 us, 256 of 1,200 700 and 559, 40 of 14,000 1,018 and 748, 20 of 5,000 209 and 186, 8 of 5,000 99
+// and 94; two turns 535 at 64 of 5,000, eight 464.  Colonies of 16 lanes gain little (16 of 30,000: 615 and
+// 574), of eight nothing.
+constexpr int PAIR32_SPLIT_SHIFT = 5, PAIR32_SPLIT = 2;  // colonies of 2^5 lanes take 2^2 turns
+__host__ __device__ inline int pair32_split_shift(int shift) {
+  return shift == PAIR32_SPLIT_SHIFT ? shift - PAIR32_SPLIT : shift;
+}
+template <int D, bool QUEUED, bool SPLIT>
 __device__ __forceinline__ void pair32_forces(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
   __shared__ int guard[256][GUARD_SLOTS];        // each lane's pairs inside the LJ guard band
   constexpr int U = QUEUED ? PAIR32_UNROLL : 2;
   // each lane's candidates in reach, not yet evaluated: sorted slot, bin offsets
   __shared__ uint2 queue[QUEUED ? PAIR32_QUEUE : 1][QUEUED ? 256 : 1];
+  // each lane's sums of 2^l shares that wait for the next 2^l
+  __shared__ float4 part[SPLIT ? PAIR32_SPLIT : 1][SPLIT ? 256 : 1];
   const StepParams& P = *Pp;
   const float4* __restrict__ spos = (const float4*)S.spos;
   const int* __restrict__ smeta = S.smeta;
@@ -1415,10 +1429,12 @@ __device__ __forceinline__ void pair32_forces(const StepParams* __restrict__ Pp,
   const int* __restrict__ start = S.start;
   const int lane = threadIdx.x & (WAVE - 1);
   const int sh = P.pair_shift, lanes = 1 << sh;
+  const int rs = SPLIT ? pair32_split_shift(sh) : sh, own = 1 << rs;  // lanes at work on a particle
+  const int extra = SPLIT ? sh - rs : 0;                              // log2 of each one's turns
   const int w = __builtin_amdgcn_readfirstlane(bid * (blockDim.x / WAVE) + threadIdx.x / WAVE);
   int tp, k0, k1;
-  if (!wave_type_chunk(P, start, w, WAVE >> sh, &tp, &k0, &k1)) return;
-  const int k = k0 + (lane >> sh), sub = lane & (lanes - 1);
+  if (!wave_type_chunk(P, start, w, WAVE >> rs, &tp, &k0, &k1)) return;
+  const int k = k0 + (lane >> rs), me_lane = lane & (own - 1);
   if (k >= k1) return;
   const uint32_t ts = (uint32_t)step_ts(S);
   const int nE = P.nE;
@@ -1444,7 +1460,7 @@ __device__ __forceinline__ void pair32_forces(const StepParams* __restrict__ Pp,
   const bool any_one = one[0] || one[1] || one[2];
   const float wr = wid[D - 1], iwr = (float)P.invw[D - 1], mr = xl[D - 1];
   float F[3] = {0.f, 0.f, 0.f}, pr = 0.f;
-  int nguard = 0, nq = 0;
+  int nguard = 0, nq = 0, guards = 0;
   // the vector from p (at qx, qy, qr of the candidate's bin frame) to a candidate
   auto delta = [&](const float4& r, float qx, float qy, float qr, float& dx, float& dy, float& dz) {
     dx = r.x - qx;
@@ -1457,162 +1473,184 @@ __device__ __forceinline__ void pair32_forces(const StepParams* __restrict__ Pp,
     }
     return fmaf(dx, dx, fmaf(dy, dy, dz * dz));
   };
-  for (int tq = 0; tq < P.ntypes; ++tq) {
-    const int Rx = P.reach_tt[tp][tq][0];
-    if (Rx < 0) continue;
-    const int Rm = D == 3 ? P.reach_tt[tp][tq][1] : 0, Rr = P.reach_tt[tp][tq][D - 1];
-    const Law32 Lw = law32(P, tp, tq);
-    const float rca = (float)P.rca_tt[tp][tq], rcb = (float)P.rcb_tt[tp][tq];
-    const float cadh = (P.cls_spec[tq] == spec_p) ? 1.0f : ca_p;  // scale for f0 >= 0 (MD.cu:345-360)
-    const bool same_species_cells = nE == 2 && (P.cls_spec[tq] == spec_p);
-    // This particle's largest cut-off against type tq (diameter bound of tq), with a margin
-    // far above FP32 rounding: bins beyond it cannot hold a partner.  Columns are culled by
-    // their x/y gap and each run is clipped to the bins its remaining radius reaches.
-    const float rcp = fmaf(rca, me.w + (float)P.sigma_bound[tq], rcb) * 1.001f + 1e-6f;
-    const float rcp2 = rcp * rcp;
-    const float rct = rca * 1.0001f, rcu = fmaf(rca, me.w, rcb) * 1.0001f;  // a candidate's cut-off, widened
-    // evaluates the lane's queued candidates, in their order
-    auto flush = [&]() {
-      for (int h = 0; h < nq; ++h) {
-        const uint2 e = queue[h][threadIdx.x];
-        const int j = (int)e.x;
-        if (j == k) continue;
-        const float4 r = spos[j];
-        if (same_species_cells && ((smeta[j] >> 3) >> cshift) == cell_p) continue;
-        const float qx = me.x - (float)((int)(e.y << 24) >> 24) * wid[0];
-        const float qy = me.y - (float)((int)(e.y << 16) >> 24) * wid[1];
-        float dx, dy, dz, f0, temp;
-        const float r2 = delta(r, qx, qy, mr - (float)((int)e.y >> 16) * wr, dx, dy, dz);
-        bool contact;
-        if (!pair_term32<D>(P, S, Lw, guard[threadIdx.x], j, pidx, me.w, r.w, r2, ts, dx, dy, nguard, f0, contact, temp)) continue;
-        const float fs = f0 < 0.0f ? f0 : cadh * f0;
-        F[0] = fmaf(fs, dx, F[0]);
-        F[1] = fmaf(fs, dy, F[1]);
-        if (D == 3) F[2] = fmaf(fs, dz, F[2]);
-        if (contact && temp != 0.0f) pr -= fs / temp;
-      }
-      nq = 0;
-    };
-    const int side = 2 * Rm + 1, ncol = (2 * Rx + 1) * side;
-    const float iside = rcp32((float)side);
-    for (int c = sub; c < ncol; c += lanes) {
-      const int cx = D == 3 ? (int)(((float)c + 0.5f) * iside) : c;  // c / side (both far below 2^20)
-      const int ox = cx - Rx, oy = D == 3 ? c - cx * side - Rm : 0;
-      int nx = bc[0] + ox;
-      if (P.box.pbc[0]) nx = nx < 0 ? nx + P.ns[0] : (nx >= P.ns[0] ? nx - P.ns[0] : nx);
-      else if (nx < 0 || nx >= P.ns[0]) continue;
-      const float qx = me.x - (float)ox * wid[0];
-      const float gx = one[0] ? 0.0f : (ox > 0 ? (float)ox * wid[0] - loc[0] : (ox < 0 ? loc[0] - (float)(ox + 1) * wid[0] : 0.0f));
-      float rem = rcp2 - (gx > 0.0f ? gx * gx : 0.0f), qy = 0.0f;
-      int row = nx;
-      if (D == 3) {
-        int ny = bc[1] + oy;
-        if (P.box.pbc[1]) ny = ny < 0 ? ny + P.ns[1] : (ny >= P.ns[1] ? ny - P.ns[1] : ny);
-        else if (ny < 0 || ny >= P.ns[1]) continue;
-        qy = me.y - (float)oy * wid[1];
-        const float gy = one[1] ? 0.0f : (oy > 0 ? (float)oy * wid[1] - loc[1] : (oy < 0 ? loc[1] - (float)(oy + 1) * wid[1] : 0.0f));
-        rem -= gy > 0.0f ? gy * gy : 0.0f;
-        row = nx * P.ns[1] + ny;
-      }
-      if (rem < 0.0f) continue;
-      int lo = -Rr, hi = Rr;
-      if (!one[D - 1]) {
-        // the radius margin (1e-3 of the cut-off) covers the rounding of the root and the reciprocal
-        const float sr = sqrt32(rem);
-        const int a = (int)floorf((loc[D - 1] + sr) * iwr), b = (int)ceilf((loc[D - 1] - sr) * iwr) - 1;
-        hi = a < Rr ? a : Rr;
-        lo = b > -Rr ? b : -Rr;
-        if (lo > hi) continue;
-      }
-      int z0[2], z1[2], zo[2];
-      const int nseg = run_segments(P, D - 1, bc[D - 1], lo, hi, z0, z1, zo);
-      const int base = tq * P.nbins + row * P.ns[D - 1];
-      const unsigned col = (unsigned)(ox & 255) | (unsigned)(oy & 255) << 8;
-      for (int sg = 0; sg < nseg; ++sg) {
-        const int unwrap = zo[sg] - z0[sg];  // bin coordinate along the run -> offset from p's bin
-        const int j1 = start[base + z1[sg] + 1];
-        for (int j = start[base + z0[sg]]; j < j1; j += U) {
-          float4 r[U];
-          int sb[U];
-          if constexpr (QUEUED) {
-            // byte offsets in 32 bits (a sorted slot is below 2^28); the arrays hold PAIR32_UNROLL
-            // records more than there are slots
-            const float4* rj = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(spos) + ((unsigned)j << 4));
-            const int* bj = reinterpret_cast<const int*>(reinterpret_cast<const char*>(sbin) + ((unsigned)j << 2));
+  for (int turn = 0; turn < (SPLIT ? 1 << extra : 1); ++turn) {
+    // the shares in bit-reversed order: neighbours in it are the tree's first pairs
+    const int sub = me_lane | (SPLIT && extra ? (int)(__brev((unsigned)turn) >> (32 - extra)) << rs : 0);
+    for (int tq = 0; tq < P.ntypes; ++tq) {
+      const int Rx = P.reach_tt[tp][tq][0];
+      if (Rx < 0) continue;
+      const int Rm = D == 3 ? P.reach_tt[tp][tq][1] : 0, Rr = P.reach_tt[tp][tq][D - 1];
+      if (SPLIT && sub >= (2 * Rx + 1) * (2 * Rm + 1)) continue;
+      const Law32 Lw = law32(P, tp, tq);
+      const float rca = (float)P.rca_tt[tp][tq], rcb = (float)P.rcb_tt[tp][tq];
+      const float cadh = (P.cls_spec[tq] == spec_p) ? 1.0f : ca_p;  // scale for f0 >= 0 (MD.cu:345-360)
+      const bool same_species_cells = nE == 2 && (P.cls_spec[tq] == spec_p);
+      // This particle's largest cut-off against type tq (diameter bound of tq), with a margin
+      // far above FP32 rounding: bins beyond it cannot hold a partner.  Columns are culled by
+      // their x/y gap and each run is clipped to the bins its remaining radius reaches.
+      const float rcp = fmaf(rca, me.w + (float)P.sigma_bound[tq], rcb) * 1.001f + 1e-6f;
+      const float rcp2 = rcp * rcp;
+      const float rct = rca * 1.0001f, rcu = fmaf(rca, me.w, rcb) * 1.0001f;  // a candidate's cut-off, widened
+      // evaluates the lane's queued candidates, in their order
+      auto flush = [&]() {
+        for (int h = 0; h < nq; ++h) {
+          const uint2 e = queue[h][threadIdx.x];
+          const int j = (int)e.x;
+          if (j == k) continue;
+          const float4 r = spos[j];
+          if (same_species_cells && ((smeta[j] >> 3) >> cshift) == cell_p) continue;
+          const float qx = me.x - (float)((int)(e.y << 24) >> 24) * wid[0];
+          const float qy = me.y - (float)((int)(e.y << 16) >> 24) * wid[1];
+          float dx, dy, dz, f0, temp;
+          const float r2 = delta(r, qx, qy, mr - (float)((int)e.y >> 16) * wr, dx, dy, dz);
+          bool contact;
+          if (!pair_term32<D>(P, S, Lw, guard[threadIdx.x], j, pidx, me.w, r.w, r2, ts, dx, dy, nguard, f0, contact, temp)) continue;
+          const float fs = f0 < 0.0f ? f0 : cadh * f0;
+          F[0] = fmaf(fs, dx, F[0]);
+          F[1] = fmaf(fs, dy, F[1]);
+          if (D == 3) F[2] = fmaf(fs, dz, F[2]);
+          if (contact && temp != 0.0f) pr -= fs / temp;
+        }
+        nq = 0;
+      };
+      const int side = 2 * Rm + 1, ncol = (2 * Rx + 1) * side;
+      const float iside = rcp32((float)side);
+      for (int c = sub; c < ncol; c += lanes) {
+        const int cx = D == 3 ? (int)(((float)c + 0.5f) * iside) : c;  // c / side (both far below 2^20)
+        const int ox = cx - Rx, oy = D == 3 ? c - cx * side - Rm : 0;
+        int nx = bc[0] + ox;
+        if (P.box.pbc[0]) nx = nx < 0 ? nx + P.ns[0] : (nx >= P.ns[0] ? nx - P.ns[0] : nx);
+        else if (nx < 0 || nx >= P.ns[0]) continue;
+        const float qx = me.x - (float)ox * wid[0];
+        const float gx = one[0] ? 0.0f : (ox > 0 ? (float)ox * wid[0] - loc[0] : (ox < 0 ? loc[0] - (float)(ox + 1) * wid[0] : 0.0f));
+        float rem = rcp2 - (gx > 0.0f ? gx * gx : 0.0f), qy = 0.0f;
+        int row = nx;
+        if (D == 3) {
+          int ny = bc[1] + oy;
+          if (P.box.pbc[1]) ny = ny < 0 ? ny + P.ns[1] : (ny >= P.ns[1] ? ny - P.ns[1] : ny);
+          else if (ny < 0 || ny >= P.ns[1]) continue;
+          qy = me.y - (float)oy * wid[1];
+          const float gy = one[1] ? 0.0f : (oy > 0 ? (float)oy * wid[1] - loc[1] : (oy < 0 ? loc[1] - (float)(oy + 1) * wid[1] : 0.0f));
+          rem -= gy > 0.0f ? gy * gy : 0.0f;
+          row = nx * P.ns[1] + ny;
+        }
+        if (rem < 0.0f) continue;
+        int lo = -Rr, hi = Rr;
+        if (!one[D - 1]) {
+          // the radius margin (1e-3 of the cut-off) covers the rounding of the root and the reciprocal
+          const float sr = sqrt32(rem);
+          const int a = (int)floorf((loc[D - 1] + sr) * iwr), b = (int)ceilf((loc[D - 1] - sr) * iwr) - 1;
+          hi = a < Rr ? a : Rr;
+          lo = b > -Rr ? b : -Rr;
+          if (lo > hi) continue;
+        }
+        int z0[2], z1[2], zo[2];
+        const int nseg = run_segments(P, D - 1, bc[D - 1], lo, hi, z0, z1, zo);
+        const int base = tq * P.nbins + row * P.ns[D - 1];
+        const unsigned col = (unsigned)(ox & 255) | (unsigned)(oy & 255) << 8;
+        for (int sg = 0; sg < nseg; ++sg) {
+          const int unwrap = zo[sg] - z0[sg];  // bin coordinate along the run -> offset from p's bin
+          const int j1 = start[base + z1[sg] + 1];
+          for (int j = start[base + z0[sg]]; j < j1; j += U) {
+            float4 r[U];
+            int sb[U];
+            if constexpr (QUEUED) {
+              // byte offsets in 32 bits (a sorted slot is below 2^28); the arrays hold PAIR32_UNROLL
+              // records more than there are slots
+              const float4* rj = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(spos) + ((unsigned)j << 4));
+              const int* bj = reinterpret_cast<const int*>(reinterpret_cast<const char*>(sbin) + ((unsigned)j << 2));
 #pragma unroll
-            for (int q = 0; q < U; ++q) {
-              r[q] = rj[q];
-              sb[q] = bj[q];
-            }
-#pragma unroll
-            for (int q = 0; q < U; ++q) {
-              const int orun = run_coord<D>(sb[q]) + unwrap;
-              float dx, dy, dz;
-              const float r2 = delta(r[q], qx, qy, mr - (float)orun * wr, dx, dy, dz);
-              const float rc = fmaf(rct, r[q].w, rcu);
-              if (j + q >= j1 || r2 > rc * rc) continue;
-              queue[nq][threadIdx.x] = make_uint2((unsigned)(j + q), col | (unsigned)orun << 16);
-              ++nq;
-            }
-            if (__any(nq > PAIR32_QUEUE - U)) flush();
-          } else {
-#pragma unroll
-            for (int q = 0; q < U; ++q) {
-              const int jj = j + q < j1 ? j + q : j1 - 1;
-              r[q] = spos[jj];
-              sb[q] = sbin[jj];
-            }
-#pragma unroll
-            for (int q = 0; q < U; ++q) {
-              const float qr = mr - (float)(run_coord<D>(sb[q]) + unwrap) * wr;
-              float dx = r[q].x - qx, dy = D == 3 ? r[q].y - qy : r[q].y - qr, dz = D == 3 ? r[q].z - qr : 0.0f;
-              if (any_one) {
-                if (one[0]) dx -= (float)P.box.L[0] * rintf(dx * (float)P.box.invL[0]);
-                if (one[1]) dy -= (float)P.box.L[1] * rintf(dy * (float)P.box.invL[1]);
-                if (D == 3 && one[2]) dz -= (float)P.box.L[2] * rintf(dz * (float)P.box.invL[2]);
+              for (int q = 0; q < U; ++q) {
+                r[q] = rj[q];
+                sb[q] = bj[q];
               }
-              const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-              const float ssum = r[q].w + me.w;
-              const float rc = fmaf(rca, ssum, rcb);
-              const int jq = j + q;
-              if (jq >= j1 || r2 > rc * rc * 1.0001f || jq == k) continue;
-              if (same_species_cells && ((smeta[jq] >> 3) >> cshift) == cell_p) continue;
-              float f0, temp;
-              bool contact;
-              if (!pair_term32<D>(P, S, Lw, guard[threadIdx.x], jq, pidx, me.w, r[q].w, r2, ts, dx, dy, nguard, f0, contact, temp)) continue;
-              const float fs = f0 < 0.0f ? f0 : cadh * f0;
-              F[0] = fmaf(fs, dx, F[0]);
-              F[1] = fmaf(fs, dy, F[1]);
-              if (D == 3) F[2] = fmaf(fs, dz, F[2]);
-              if (contact && temp != 0.0f) pr -= fs / temp;
+#pragma unroll
+              for (int q = 0; q < U; ++q) {
+                const int orun = run_coord<D>(sb[q]) + unwrap;
+                float dx, dy, dz;
+                const float r2 = delta(r[q], qx, qy, mr - (float)orun * wr, dx, dy, dz);
+                const float rc = fmaf(rct, r[q].w, rcu);
+                if (j + q >= j1 || r2 > rc * rc) continue;
+                queue[nq][threadIdx.x] = make_uint2((unsigned)(j + q), col | (unsigned)orun << 16);
+                ++nq;
+              }
+              if (__any(nq > PAIR32_QUEUE - U)) flush();
+            } else {
+#pragma unroll
+              for (int q = 0; q < U; ++q) {
+                const int jj = j + q < j1 ? j + q : j1 - 1;
+                r[q] = spos[jj];
+                sb[q] = sbin[jj];
+              }
+#pragma unroll
+              for (int q = 0; q < U; ++q) {
+                const float qr = mr - (float)(run_coord<D>(sb[q]) + unwrap) * wr;
+                float dx = r[q].x - qx, dy = D == 3 ? r[q].y - qy : r[q].y - qr, dz = D == 3 ? r[q].z - qr : 0.0f;
+                if (any_one) {
+                  if (one[0]) dx -= (float)P.box.L[0] * rintf(dx * (float)P.box.invL[0]);
+                  if (one[1]) dy -= (float)P.box.L[1] * rintf(dy * (float)P.box.invL[1]);
+                  if (D == 3 && one[2]) dz -= (float)P.box.L[2] * rintf(dz * (float)P.box.invL[2]);
+                }
+                const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                const float ssum = r[q].w + me.w;
+                const float rc = fmaf(rca, ssum, rcb);
+                const int jq = j + q;
+                if (jq >= j1 || r2 > rc * rc * 1.0001f || jq == k) continue;
+                if (same_species_cells && ((smeta[jq] >> 3) >> cshift) == cell_p) continue;
+                float f0, temp;
+                bool contact;
+                if (!pair_term32<D>(P, S, Lw, guard[threadIdx.x], jq, pidx, me.w, r[q].w, r2, ts, dx, dy, nguard, f0, contact, temp)) continue;
+                const float fs = f0 < 0.0f ? f0 : cadh * f0;
+                F[0] = fmaf(fs, dx, F[0]);
+                F[1] = fmaf(fs, dy, F[1]);
+                if (D == 3) F[2] = fmaf(fs, dz, F[2]);
+                if (contact && temp != 0.0f) pr -= fs / temp;
+              }
             }
           }
         }
       }
+      if (QUEUED) flush();
     }
-    if (QUEUED) flush();
-  }
-  if (nguard > 0) {
-    float g[3] = {0.f, 0.f, 0.f};
-    guard_force(P, S, k, guard[threadIdx.x], nguard, g);
-    for (int d = 0; d < D; ++d) F[d] += g[d];
+    if (nguard > 0) {
+      float g[3] = {0.f, 0.f, 0.f};
+      guard_force(P, S, k, guard[threadIdx.x], nguard, g);
+      for (int d = 0; d < D; ++d) F[d] += g[d];
+    }
+    guards += nguard;
+    if constexpr (SPLIT) {
+      nguard = 0;
+      const int ones = min(__ffs(~turn) - 1, extra);  // complete levels below the sum that now waits
+      for (int l = 0; l < ones; ++l) {
+        const float4 x = part[l][threadIdx.x];
+        F[0] += x.x, F[1] += x.y, F[2] += x.z, pr += x.w;
+      }
+      if (ones < extra) {
+        part[ones][threadIdx.x] = make_float4(F[0], F[1], F[2], pr);
+        F[0] = F[1] = F[2] = pr = 0.f;
+      }
+    }
   }
   float* fp = (float*)S.fpair;
 #pragma unroll
   for (int d = 0; d < D; ++d) {
-    const float f = group_sum(F[d], lanes);
-    if (sub == 0) fp[(size_t)d * S.P + k] = f;
+    const float f = group_sum(F[d], own);
+    if (me_lane == 0) fp[(size_t)d * S.P + k] = f;
   }
   if (P.pressure) {
-    pr = group_sum(pr, lanes);
-    if (sub == 0) ((float*)S.ppair)[k] = pr;
+    pr = group_sum(pr, own);
+    if (me_lane == 0) ((float*)S.ppair)[k] = pr;
   }
-  if (group_sum(nguard, lanes) > GUARD_SLOTS) atomicOr(S.err, (unsigned)ERR_GUARD);
+  if (group_sum(guards, own) > GUARD_SLOTS) atomicOr(S.err, (unsigned)ERR_GUARD);
 }
 template <int D, bool QUEUED>
 __device__ inline void k_pair32_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
-  pair32_forces<D, QUEUED>(Pp, S, bid);
+  pair32_forces<D, QUEUED, false>(Pp, S, bid);
   clear_counts(*Pp, S, bid * (int)blockDim.x + (int)threadIdx.x, S.P << Pp->pair_shift);
+}
+__device__ inline void k_pair32_split_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
+  pair32_forces<3, false, true>(Pp, S, bid);
+  clear_counts(*Pp, S, bid * (int)blockDim.x + (int)threadIdx.x, S.P << pair32_split_shift(Pp->pair_shift));
 }
 #define PAIR32_WPE 5  // six waves per SIMD spill
 template <int D, bool QUEUED>

@@ -250,3 +250,41 @@ def test_generic_kernel_passes(gpu, capacity):
     d -= 14.0 * np.round(d / 14.0)
     # 12 steps of dt 1e-4: FP32 force errors of 1e-5 of forces up to a few hundred move a disc by 1e-5
     assert np.max(np.abs(d)) <= 1e-5
+
+
+@pytest.mark.parametrize("caps", [(500, 16000, 33000, 70000), (16384, 16384, 12001, 16384, 16384),
+                                  (16384, 16384, 16384, 16384, 16383, 20000, 40000, 300000)])
+@pytest.mark.parametrize("law", ["lj", abi.LAW_HZ])
+def test_batched_3d_members_keep_their_bits(gpu, law, caps):
+    """3D FP32 colonies in a batch against the same alone: evaluated at once where the colony alone queues
+    (over 32,768 slots), and in turns by fewer lanes where colonies of 32 lanes overfill the chip (over 65,536
+    slots together)."""
+    members, ends = [], []
+    for c, cap in enumerate(caps):
+        if law == "lj":
+            p, box, col = configs.relaxed_bulk_3d(400, seed=c, precision=abi.PREC_FP32)
+        else:
+            p, box, col = _colony(3, 380 + c, 7.0, c & 1, law, cap, 40 + c)
+            p.precision, p.dt = abi.PREC_FP32, 1e-5
+        n = [sp["ncells"] for sp in col.species]
+        room = [cap - n[1], n[1]]
+        alone = HipMD(p, box, room)
+        both = [alone, HipMD(p, box, room)]
+        for md in both:
+            md.upload(col)
+            md.forces(want=False)
+        members.append(both[1])
+        alone.step(11, 0)
+        end = Colony(3, 1, room)
+        alone.download(end)
+        alone.close()
+        ends.append(end)
+    batch = HipBatch(members)
+    batch.step(11, [0] * len(caps))
+    batch.close()
+    for md, end in zip(members, ends):
+        got = Colony(3, 1, [sp["capacity"] for sp in end.species])
+        md.download(got)
+        md.close()
+        for f in ("pos", "vel", "frc", "pressure"):
+            assert np.array_equal(got.flat(f), end.flat(f)), (f, end.species[0]["capacity"])
