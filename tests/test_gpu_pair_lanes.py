@@ -39,7 +39,7 @@ def _colony(dim, n, L, periodic, law, capacity, seed, stray=0):
     return p, box, col
 
 
-def _worst(p, box, col, tol, floor, skin=0.0):
+def _worst(p, box, col, tol, floor, skin=0.0, extra=0):
     dim = p.dim
     q = abi.Params.from_buffer_copy(p)
     q.precision = abi.PREC_FP64
@@ -48,7 +48,7 @@ def _worst(p, box, col, tol, floor, skin=0.0):
     orc.forces(ref, 0)
     scale = orc.force_scale(ref)
     orc.close()
-    md = HipMD(p, box, [sp["capacity"] for sp in col.species])
+    md = HipMD(p, box, [extra + sp["capacity"] for sp in col.species])
     md.upload(col)
     if skin:
         md.set_neighbour_list(True, skin, 1024)
@@ -106,7 +106,7 @@ def test_list_lanes(gpu, cap, law):
 @pytest.mark.parametrize("cap", LIST_CAPS)
 def test_two_level_list_lanes(gpu, cap):
     """The inner list keeps each lane's entries and their order: bit-identical to one level, through
-    refreshes and rebuilds; and the capacity is the particle's, whatever the lanes."""
+    refreshes and rebuilds."""
     p, box, col = configs.relaxed_bulk_3d(4096, seed=3, precision=abi.PREC_FP32)
     ends = []
     for inner in (0.0, 0.05):
@@ -121,22 +121,29 @@ def test_two_level_list_lanes(gpu, cap):
         ends.append(c)
     for f in ("pos", "vel", "frc"):
         assert np.array_equal(ends[0].flat(f), ends[1].flat(f)), f
-    codes = []
-    for slots in (48, 52, 56, 60, 64, 68, 72, 76, 80, 84, 88, 92, 96, 100, 104, 108, 112, 116, 120):
-        md = HipMD(p, box, [cap + sp["capacity"] for sp in col.species])
-        md.upload(col)
-        md.set_neighbour_list(True, 0.15, slots)
-        try:
-            md.forces(want=False)
-            codes.append(slots)
-        except abi.CilError as e:
-            assert e.code == -3
-        md.close()
-    _SMALLEST.setdefault("slots", codes[0])
-    assert codes[0] == _SMALLEST["slots"] and codes == list(range(codes[0], 121, 4))
 
 
-_SMALLEST = {}
+def test_list_capacity_is_the_particles(gpu):
+    """The smallest list capacity that holds a colony is the same at eight, four, two and one lane per
+    particle, and every larger one holds it."""
+    p, box, col = configs.relaxed_bulk_3d(4096, seed=3, precision=abi.PREC_FP32)
+    slots = list(range(48, 121, 4))
+    accepted = []
+    for cap in LIST_CAPS:
+        codes = []
+        for n in slots:
+            md = HipMD(p, box, [cap + sp["capacity"] for sp in col.species])
+            md.upload(col)
+            md.set_neighbour_list(True, 0.15, n)
+            try:
+                md.forces(want=False)
+                codes.append(n)
+            except abi.CilError as e:
+                assert e.code == -3
+            md.close()
+        accepted.append(codes)
+    assert all(a == accepted[0] for a in accepted) and slots[0] < accepted[0][0]
+    assert accepted[0] == list(range(accepted[0][0], 121, 4))
 
 
 @pytest.mark.parametrize("mode", ["fp64", "fp32", "list32"])
@@ -288,3 +295,65 @@ def test_batched_3d_members_keep_their_bits(gpu, law, caps):
         md.close()
         for f in ("pos", "vel", "frc", "pressure"):
             assert np.array_equal(got.flat(f), end.flat(f)), (f, end.species[0]["capacity"])
+
+
+def _cutoff_pairs(seed):
+    """The relaxed LJ / soft-core bulk with 60 disjoint LJ pairs moved to 1 +- 5e-6 .. 1e-10 of their cut-off,
+    where FP32 distances cannot tell inside from outside."""
+    p, box, col = configs.relaxed_bulk_3d(1200, seed=seed, precision=abi.PREC_FP32)
+    L, rng = box.length[0], np.random.default_rng(seed)
+    x, sig = col.species[0]["pos"][:, 0], col.species[0]["sigma"][:, 0]
+    left, done = set(range(len(x))), 0
+    for i in rng.permutation(len(x)):
+        if i not in left or done == 60:
+            continue
+        d = x - x[i]
+        d -= L * np.round(d / L)
+        r, rc = np.linalg.norm(d, axis=1), 2.5 * 0.5 * (sig + sig[i])
+        near = [j for j in np.nonzero(np.abs(r / rc - 1) < 0.01)[0] if j in left]
+        if not near:
+            continue
+        j = near[0]
+        delta = (1, -1)[done % 2] * (5e-6, 1e-7, 1e-10)[done % 3]
+        x[j] = np.mod(x[i] + d[j] * (rc[j] * (1 + delta) / r[j]), L)
+        left -= {i, j}
+        done += 1
+    assert done == 60
+    return p, box, col
+
+
+@pytest.mark.parametrize("mode", ["stencil", "list"])
+@pytest.mark.parametrize("extra", [0, 10000, 20000, 50000, 130000, 300000])
+def test_lj_cutoff_band(gpu, mode, extra):
+    """FP32 LJ forces at every number of lanes, evaluated at once (extra slots up to 10,000 in each of two
+    species) and from queues, and over lists, with pairs on the cut-off: their FP64 decision is the oracle's.
+    A pair decided wrongly is off by the LJ force at the cut-off, 0.04: more than the bar of a particle whose
+    terms sum to less than 4,000."""
+    p, box, col = _cutoff_pairs(7)
+    worst, _, _ = _worst(p, box, col, 1e-5, 0.01, skin=0.3 if mode == "list" else 0.0, extra=extra)
+    assert worst <= 1.0, worst
+
+
+@pytest.mark.parametrize("mode", ["stencil", "list"])
+@pytest.mark.parametrize("extra", [0, 20000, 50000, 130000, 300000])
+@pytest.mark.parametrize("partners", [4, 5])
+def test_cutoff_band_limit_is_the_particles(gpu, mode, extra, partners):
+    """Four pairs on the cut-off of one particle are decided, five reported, whatever the lanes."""
+    p, box, _ = configs.bulk_3d_mixed(n=64, seed=1)
+    for d in range(3):
+        box.length[d] = 12.0
+    u = np.array([[1, 0, 0], [-1, 0, 0], [0, 1, 0], [0, -1, 0], [0, 0, 1]])[:partners]
+    col = Colony(3, 1, [8 + extra, 8], ncells=[1 + partners, 0])
+    col.species[0]["pos"][:1 + partners, 0] = np.concatenate([[[6, 6, 6]], 6 + 2.5 * (1 + 1e-7) * u])
+    col.species[0]["sigma"][:] = 1.0
+    md = HipMD(p, box, [sp["capacity"] for sp in col.species])
+    md.upload(col)
+    if mode == "list":
+        md.set_neighbour_list(True, 0.3, 64)
+    if partners == 4:
+        md.forces()
+    else:
+        with pytest.raises(abi.CilError) as e:
+            md.forces()
+        assert "guard-band" in str(e.value)
+    md.close()
