@@ -1399,7 +1399,7 @@ __device__ __forceinline__ int run_coord(int sb) { return D == 3 ? (sb & 1023) :
 // immediate and queued: 4,001 particles 33 and 37 us (32 lanes), 30,011 66 and 66 (16), 64,011 102 and
 // 96 (8), 131,071 174 and 158 (4), 300,011 340 and 325, 1,000,003 830 and 752 (1); 32 two-disc 2D
 // colonies at once 87 and 95.
-constexpr int PAIR32_UNROLL = 4;  // candidates per pass, at most: 4 in 3D, 2 in 2D
+constexpr int PAIR32_UNROLL = 4;  // candidates per pass where they are queued; 2 where they are evaluated at once
 constexpr int PAIR32_QUEUE = 12;
 constexpr int PAIR32_QUEUE_SHIFT = 3;  // queued up to 2^3 lanes per particle
 // SPLIT (batches of small 3D colonies, choose_lane_split): a lane takes the shares of four of the 32 lanes that
@@ -1407,9 +1407,9 @@ constexpr int PAIR32_QUEUE_SHIFT = 3;  // queued up to 2^3 lanes per particle
 // forces have the bits of the colony alone.  Alone, a colony of 5,000 needs the 32 lanes to fill the chip
 // (46 us a step against 260 with one); a batch fills it anyway, and lanes on different columns of one
 // particle wait for the longest column.  Step, 32 lanes at once and 8 in four turns: 64 colonies of 5,000 608
-// and 478 us, 256 of 1,200 700 and 559, 40 of 14,000 1,018 and 748, 20 of 5,000 209 and 186, 8 of 5,000 99
-// and 94; two turns 535 at 64 of 5,000, eight 464.  Colonies of 16 lanes gain little (16 of 30,000: 615 and
-// 574), of eight nothing.
+// and 437 us, 256 of 1,200 700 and 520, 40 of 14,000 1,018 and 678, 20 of 5,000 209 and 171.  (With more
+// registers spilled: two, four and eight turns 535, 478 and 464 at 64 of 5,000; colonies of 16 lanes gained
+// little, 16 of 30,000 615 and 574, and of eight nothing.)
 constexpr int PAIR32_SPLIT_SHIFT = 5, PAIR32_SPLIT = 2;  // colonies of 2^5 lanes take 2^2 turns
 __host__ __device__ inline int pair32_split_shift(int shift) {
   return shift == PAIR32_SPLIT_SHIFT ? shift - PAIR32_SPLIT : shift;
@@ -1460,7 +1460,7 @@ __device__ __forceinline__ void pair32_forces(const StepParams* __restrict__ Pp,
   const bool any_one = one[0] || one[1] || one[2];
   const float wr = wid[D - 1], iwr = (float)P.invw[D - 1], mr = xl[D - 1];
   float F[3] = {0.f, 0.f, 0.f}, pr = 0.f;
-  int nguard = 0, nq = 0, guards = 0;
+  int nguard = 0, nq = 0;
   // the vector from p (at qx, qy, qr of the candidate's bin frame) to a candidate
   auto delta = [&](const float4& r, float qx, float qy, float qr, float& dx, float& dy, float& dz) {
     dx = r.x - qx;
@@ -1473,9 +1473,8 @@ __device__ __forceinline__ void pair32_forces(const StepParams* __restrict__ Pp,
     }
     return fmaf(dx, dx, fmaf(dy, dy, dz * dz));
   };
-  for (int turn = 0; turn < (SPLIT ? 1 << extra : 1); ++turn) {
-    // the shares in bit-reversed order: neighbours in it are the tree's first pairs
-    const int sub = me_lane | (SPLIT && extra ? (int)(__brev((unsigned)turn) >> (32 - extra)) << rs : 0);
+  // the share of the colony's lane `sub`, added to F, pr and nguard
+  auto share = [&](int sub) __attribute__((always_inline)) {
     for (int tq = 0; tq < P.ntypes; ++tq) {
       const int Rx = P.reach_tt[tp][tq][0];
       if (Rx < 0) continue;
@@ -1617,8 +1616,13 @@ __device__ __forceinline__ void pair32_forces(const StepParams* __restrict__ Pp,
       guard_force(P, S, k, guard[threadIdx.x], nguard, g);
       for (int d = 0; d < D; ++d) F[d] += g[d];
     }
-    guards += nguard;
-    if constexpr (SPLIT) {
+  };
+  if constexpr (SPLIT) {
+    int guards = 0;
+    for (int turn = 0; turn < 1 << extra; ++turn) {
+      // the shares in bit-reversed order: neighbours in it are the tree's first pairs
+      share(me_lane | (extra ? (int)(__brev((unsigned)turn) >> (32 - extra)) << rs : 0));
+      guards += nguard;
       nguard = 0;
       const int ones = min(__ffs(~turn) - 1, extra);  // complete levels below the sum that now waits
       for (int l = 0; l < ones; ++l) {
@@ -1630,6 +1634,9 @@ __device__ __forceinline__ void pair32_forces(const StepParams* __restrict__ Pp,
         F[0] = F[1] = F[2] = pr = 0.f;
       }
     }
+    nguard = guards;
+  } else {
+    share(me_lane);
   }
   float* fp = (float*)S.fpair;
 #pragma unroll
@@ -1641,7 +1648,7 @@ __device__ __forceinline__ void pair32_forces(const StepParams* __restrict__ Pp,
     pr = group_sum(pr, own);
     if (me_lane == 0) ((float*)S.ppair)[k] = pr;
   }
-  if (group_sum(guards, own) > GUARD_SLOTS) atomicOr(S.err, (unsigned)ERR_GUARD);
+  if (group_sum(nguard, own) > GUARD_SLOTS) atomicOr(S.err, (unsigned)ERR_GUARD);
 }
 template <int D, bool QUEUED>
 __device__ inline void k_pair32_body(const StepParams* __restrict__ Pp, const Dev& S, int bid) {
@@ -2071,7 +2078,7 @@ __device__ __forceinline__ void list_segment(const StepParams& P, const Dev& S, 
 // Pair forces over the neighbour list (every step), after rebuilding the particle's list when
 // this pass's rebuild flag is set.  Same law code, exclusions, guard band and per-type wave
 // layout as k_pair32.  List groups are addressed with 32-bit byte offsets
-// (list_max * P * 4 < 2^32, checked by the host).
+// (list_max * (P << SH) * 4 < 2^32: choose_list_shift).
 template <int D, int SH>
 __device__ inline void k_pair_list_body(const StepParams* __restrict__ Pp, const Dev& S) {
   const StepParams& P = *Pp;
